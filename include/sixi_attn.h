@@ -121,7 +121,8 @@ typedef struct sixi_attn_params {
     float max_bias;         /* ALiBi; 0 = off                                              */
     float logit_softcap;    /* 0 = off                                                     */
     float reserved_f;
-    void* workspace;        /* device scratch of >= sixi_attn_workspace_bytes() bytes,
+    void* workspace;        /* device scratch of >= sixi_attn_workspace_bytes() bytes
+                               (or the least of sixi_attn_workspace_range()),
                                256-byte aligned; its contents need no initialisation       */
     size_t workspace_bytes;
     void* stream;           /* hipStream_t; NULL = the null stream                         */
@@ -159,6 +160,14 @@ int sixi_attn_forward_noalloc(const sixi_attn_params* p);
 /* Workspace the call needs for this description (depends on S, H, Hkv, D, n_q, n_kv and
  * the device's CU count; not on the device-side lengths). */
 int sixi_attn_workspace_bytes(const sixi_attn_params* p, size_t* bytes);
+
+/* The least workspace the call runs with, beside the size above.  The two differ for prefill-sized
+ * blocks too few to fill the GPU, over a long cache: with the full size several work-groups share
+ * the cells of each row block and leave f32 sums in the workspace (at most 16 per row block and two
+ * launch rounds, whatever the cache length), with less fewer do, down to none.  The workspace is the
+ * call's own while it runs, so calls that may overlap need one each; a call given only `least` bytes
+ * of an f16 cache's prefill writes none of it. */
+int sixi_attn_workspace_range(const sixi_attn_params* p, size_t* least, size_t* bytes);
 
 /* Host-side validation only (no device access): SIXI_OK or the error forward() returns. */
 int sixi_attn_validate(const sixi_attn_params* p);

@@ -69,6 +69,7 @@ struct FaArgs {
     int32_t seg_cost;      // tiles' worth of work charged to each segment in the split
     int64_t slot_floats;   // floats per partial slot
     int32_t* seg_pieces;   // per segment: logical work-groups of its first and last piece
+    int32_t pf_split;      // prefill: work-groups that share the cells of each row block (>= 1)
     int32_t q_q8;          // prefill over an f16-staged q8_0 cache: convert Q to the q8_0 dot type
                            // in the kernel (ggml's rule), as the q8_0 kernels do
 
@@ -184,6 +185,17 @@ constexpr int64_t kMaskPrepassMaxRows = 16384;
 // Cells of a single-stream, single-row call's mask row that every work-group of the dual
 // kernels reads itself instead of a pre-pass launch (single-stream decode).
 constexpr int64_t kMaskInlineMaxCells = 16384;
+
+// ---- prefill ----
+constexpr int kPrefillRows = 128;  // rows (block rows x heads of a kv-head) per work-group
+constexpr int kPrefillCells = 64;  // cells per tile
+// Row blocks of one (stream, kv-head).
+constexpr int prefill_row_blocks(int64_t n_q, int G) { return (int)((n_q * G + kPrefillRows - 1) / kPrefillRows); }
+// Floats of one work-group's share of a split row block: O rows, m and l.
+constexpr int prefill_slot_floats(int head_dim) { return kPrefillRows * (head_dim + 2); }
+// Work-groups that fit a CU (LDS).
+constexpr int prefill_groups_per_cu(int head_dim) { return head_dim == 128 ? 2 : 1; }
+int prefill_split(int64_t blocks, int64_t n_kv, int head_dim, int cu_count);
 
 inline int64_t decode_slot_floats(int row_tiles, int head_dim) {
     // O/l rows [16*row_tiles][head_dim] f16 (head_dim/2 floats' worth), then m and l per row

@@ -1,10 +1,14 @@
 // fa_prefill.hip -- chunked causal prefill (and any block of more than 96 rows per GQA group)
 // on gfx950 f16 MFMA (head_dim 128 and 256 over f16 KV; head_dim 128 over q8_0 KV).
 //
-// Work decomposition.  One work-group computes 128 consecutive rows (block rows j) of one
-// q-head of one stream, over every KV cell those rows see.  The grid is ordered heaviest
-// row block first (the last rows of a causal chunk see the most cells), so the long blocks
-// start first and the short ones fill in behind them.  Four waves own 32 rows each.
+// Work decomposition.  One work-group computes 128 consecutive rows of one kv-head of one stream
+// (the G q-heads of a block row lie next to each other: row r is block row r / G, head r % G of
+// the group, so a short block fills its tiles and the heads share the K/V reads), over every KV
+// cell those rows see.  The grid is ordered heaviest row block first (the last rows of a causal
+// chunk see the most cells), so the long blocks start first and the short ones fill in behind
+// them.  Four waves own 32 rows each.  Where the row blocks leave CUs idle, C work-groups share
+// the cells of each (a.pf_split, prefill_split), leave their sums in the workspace, and
+// prefill_merge adds them up.
 //
 // Per 64-cell KV tile (double-buffered in LDS, one barrier per tile), both K and V arrive by
 // direct global->LDS loads issued one tile ahead:
@@ -47,7 +51,7 @@
 namespace sixi {
 namespace {
 
-constexpr int kBM = 128;           // rows per work-group
+constexpr int kBM = kPrefillRows;  // rows per work-group
 constexpr int kBN = 64;            // cells per KV tile
 constexpr int kThreads = 256;      // 4 waves x 32 rows
 // Per head dim D: ROW-byte rows, KS k-steps of 16 dims, DB output blocks of 32 dims; a tile of
@@ -60,6 +64,13 @@ struct PfDim {
     static constexpr int GROUPS = D == 128 ? 2 : 1;   // work-groups per CU (LDS: 4 tiles each)
 };
 constexpr float kLazyLog2 = 8.0f;
+
+// A split item's share in the workspace: O [kBM][D] (plain sums), then m and l per row, in f32.
+template <int D>
+struct PrefillSlot {
+    static constexpr int M = kBM * D, L = M + kBM, FLOATS = L + kBM;
+    static_assert(FLOATS == prefill_slot_floats(D), "the dispatcher sizes the workspace by it");
+};
 
 enum { MODE_FAST = 0, MODE_GENERIC = 1, MODE_MASK = 2 };
 constexpr int kMaskWave = 32 * kBN * 2;  // bytes of one wave's mask rows of a tile (f16)
@@ -115,7 +126,7 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
     // next ones (up to n_cu more) join the earliest of them, where both run slower than a
     // work-group alone on its CU; so the heaviest ranks go to the positions that keep a CU to
     // themselves, the next ranks to the positions that will be joined, the lightest last.
-    const int SH = a.S * a.H;
+    const int per_rb = a.S * a.Hkv * a.pf_split;  // work-groups of one row block
     const int b = blockIdx.x;
     const int N = gridDim.x;
     int rank = b;
@@ -125,25 +136,31 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
         if (b < npair) rank = alone + b;
         else if (b < n_cu) rank = b - npair;
     }
-    const int rb = nrb - 1 - rank / SH;
-    const int s = (rank % SH) / a.H;
-    const int h = (rank % SH) % a.H;
-    const int g = h / a.G;
+    const int rb = nrb - 1 - rank / per_rb;
+    const int chunk = rank % per_rb / (a.S * a.Hkv);
+    const int s = rank % (a.S * a.Hkv) / a.Hkv;
+    const int g = rank % a.Hkv;
     const StreamDims sd = stream_dims(a, s);
-    const int j0 = rb * kBM;
-    if (j0 >= sd.ql) return;
-    const int j_last = min(j0 + kBM, sd.ql) - 1;
-    const int j = j0 + 32 * w + rl;  // this lane's row
-    const bool row_ok = j < sd.ql;
+    const int r0 = rb * kBM;                  // first row (of the kv-head's ql * G) of the group
+    const int n_rows = sd.ql * a.G;
+    if (r0 >= n_rows) return;
+    const int j0 = r0 / a.G;                  // block rows of the group's first and last row
+    const int j_last = min((r0 + kBM - 1) / a.G, sd.ql - 1);
+    const bool row_ok = r0 + 32 * w + rl < n_rows;
+    const int row = row_ok ? r0 + 32 * w + rl : r0;  // this lane's row (past the block: the first)
+    const int j = row / a.G;
+    const int h = g * a.G + row % a.G;
 
     // cells each row sees; tiles below t_full are unmasked for every row of the group
-    const int vis = causal ? sd.kl + min(j, j_last) + 1 : sd.nc;
+    const int vis = causal ? sd.kl + j + 1 : sd.nc;
     const int vis_max = causal ? sd.kl + j_last + 1 : sd.nc;
     const int vis_min = causal ? sd.kl + j0 + 1 : sd.nc;
     const int n_tiles = (vis_max + kBN - 1) / kBN;
     const int t_full = (MODE == MODE_GENERIC) ? 0 : vis_min / kBN;
     constexpr bool RAW = MODE != MODE_GENERIC;  // scores in raw dot-product units
-    const int t_beg = 0, t_end = n_tiles;  // the tiles walked
+    // the tiles walked: all of them, or (split) this work-group's share
+    const int t_beg = (int)((int64_t)n_tiles * chunk / a.pf_split);
+    const int t_end = (int)((int64_t)n_tiles * (chunk + 1) / a.pf_split);
 
     // ---- Q^T B operands in registers: lane l -> row j, dims 16ks + 8*hl .. +7 ----
     // (every load issued before any is used; rows past the block read its first row)
@@ -152,7 +169,7 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
         // ggml's conversion of Q to the q8_0 dot type: per 32-dim block (ks = 2bq, 2bq + 1 of
         // lanes l and l^32) d = amax/127, q = round-half-away(x * 127/amax) clamped to +-127,
         // and the MFMA takes f16(q * f16(d))
-        const char* src = a.q + (int64_t)(row_ok ? j : j0) * a.q_nb1 + (int64_t)h * a.q_nb2 + (int64_t)s * a.q_nb3;
+        const char* src = a.q + (int64_t)j * a.q_nb1 + (int64_t)h * a.q_nb2 + (int64_t)s * a.q_nb3;
         float xq[P::KS][8];
         if (a.q_f16) {
             u32x4 raw[P::KS];
@@ -198,7 +215,7 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
             }
         }
     } else {
-        const char* src = a.q + (int64_t)(row_ok ? j : j0) * a.q_nb1 + (int64_t)h * a.q_nb2 + (int64_t)s * a.q_nb3;
+        const char* src = a.q + (int64_t)j * a.q_nb1 + (int64_t)h * a.q_nb2 + (int64_t)s * a.q_nb3;
         if (a.q_f16) {
             u32x4 raw[P::KS];
 #pragma unroll
@@ -270,7 +287,7 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
         for (int db = 0; db < P::DB; ++db) vtr[db] = lds0 + kVBase + (base ^ (64u * db));
     }
 
-    PageIds pages = page_ids_load(a, s, 0);
+    PageIds pages = page_ids_load(a, s, (t_beg * kBN) >> 8);
     auto issue_kv = [&](int t, int buf) {
         const int page = t * kBN < sd.nc ? page_id(pages, a, s, (t * kBN) >> 8) : 0;
         const KvSpan ksp = kv_span(a, a.k, a.k_nb1, a.k_nb2, a.k_nb3, s, g, t * kBN, sd.nc, rowb, page);
@@ -426,7 +443,7 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
     const float slope = (MODE == MODE_GENERIC) ? alibi_slope(a, h) : 1.0f;
     const char* mrow = nullptr;
     if (MODE == MODE_GENERIC && a.mask)
-        mrow = a.mask + (int64_t)(s % a.m_ne3) * a.m_nb3 + (int64_t)min(j, j_last) * a.m_nb1;
+        mrow = a.mask + (int64_t)(s % a.m_ne3) * a.m_nb3 + (int64_t)j * a.m_nb1;
     const f32x16 zero16 = {};
 
     // MODE_MASK: the stream's mask rows through a range-checked resource (exactly its n_q rows);
@@ -442,7 +459,7 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int r = 8 * u + lane / 8;
-            const int jr = min(j0 + 32 * w + r, j_last);
+            const int jr = min((r0 + 32 * w + r) / a.G, j_last);
             mdo[u] = (uint32_t)((int64_t)jr * a.m_nb1) + 16u * (uint32_t)((lane % 8) ^ ((r >> 1) & 7));
         }
     }
@@ -674,27 +691,88 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
         if (t + 1 < t_end) run_tile(t + 1, std::integral_constant<int, 1>{});
     }
 
-    // ---- normalise and write: lane holds dims 32db + 8b + 4hl .. +3 of row j ----
+    // ---- write: lane holds dims 32db + 8b + 4hl .. +3 of its row ----
     {
         auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_sum), __float_as_uint(l_sum), false, false);
         l_sum = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
     }
-    if (row_ok) {
-        // (the row and its address are recomputed from the lane here rather than held across
-        // the tile loop)
-        int lx = lane;
-        asm volatile("" : "+v"(lx));
-        const int jw = j0 + 32 * wq + (lx & 31), hw = lx >> 5;
+    // (the row and its address are recomputed from the lane here rather than held across the
+    // tile loop)
+    int lx = lane;
+    asm volatile("" : "+v"(lx));
+    const int hw = lx >> 5;
+    const int rw = 32 * wq + (lx & 31);  // row in the group
+    if (a.pf_split > 1) {
+        // a split item: this share's plain sums and their exponent reference (log2 units)
+        if (r0 + rw >= n_rows) return;
+        float* slot = a.part + (int64_t)(chunk + a.pf_split * (g + a.Hkv * (s + a.S * rb))) * PrefillSlot<D>::FLOATS;
+        char* dst = reinterpret_cast<char*>(slot + rw * D);
+#pragma unroll
+        for (int db = 0; db < P::DB; ++db)
+#pragma unroll
+            for (int bq = 0; bq < 4; ++bq)
+                st16(dst + (32 * db + 8 * bq + 4 * hw) * 4,
+                     f32x4{acc[db][4 * bq], acc[db][4 * bq + 1], acc[db][4 * bq + 2], acc[db][4 * bq + 3]});
+        if (hw == 0) {
+            slot[PrefillSlot<D>::M + rw] = RAW ? m_ref * c2 : m_ref;
+            slot[PrefillSlot<D>::L + rw] = l_sum;
+        }
+    } else if (r0 + rw < n_rows) {
+        const int jw = (r0 + rw) / a.G, hd = g * a.G + (r0 + rw) % a.G;
         const float inv = l_sum == 0.0f ? 0.0f : 1.0f / l_sum;
-        char* dst = a.out + (int64_t)jw * a.o_nb2 + (int64_t)h * a.o_nb1 + (int64_t)s * a.o_nb3;
+        char* dst = a.out + (int64_t)jw * a.o_nb2 + (int64_t)hd * a.o_nb1 + (int64_t)s * a.o_nb3;
 #pragma unroll
         for (int db = 0; db < P::DB; ++db)
 #pragma unroll
             for (int bq = 0; bq < 4; ++bq)
                 st16(dst + (32 * db + 8 * bq + 4 * hw) * 4,
                      gated(a, f32x4{acc[db][4 * bq], acc[db][4 * bq + 1], acc[db][4 * bq + 2], acc[db][4 * bq + 3]} * inv,
-                           gate_load(a, s, jw, h, 32 * db + 8 * bq + 4 * hw)));
+                           gate_load(a, s, jw, hd, 32 * db + 8 * bq + 4 * hw)));
     }
+}
+
+// Adds up the shares of split items: out = sum_c w_c O_c / sum_c w_c l_c with w_c = 2^(m_c - max m).
+// One thread per four dims of a row; a share that saw no cell of the row has m = -inf and zero sums.
+// Moves bytes only: C x 4 D read and 4 D written per row.
+template <int D>
+__global__ __launch_bounds__(kThreads) void prefill_merge(FaArgs a) {
+    constexpr int TPR = D / 4, RPB = kThreads / TPR;  // threads per row, rows per work-group
+    constexpr int kU = 4;                             // shares whose loads are issued together
+    const int item = blockIdx.x / (kBM / RPB);
+    const int rw = (int)(blockIdx.x % (kBM / RPB)) * RPB + (int)threadIdx.x / TPR;
+    const int d = 4 * ((int)threadIdx.x % TPR);
+    const int g = item % a.Hkv, s = item / a.Hkv % a.S, rb = item / (a.Hkv * a.S);
+    const StreamDims sd = stream_dims(a, s);
+    const int r = rb * kBM + rw;
+    if (r >= sd.ql * a.G) return;
+    const float* slot = a.part + (int64_t)item * a.pf_split * PrefillSlot<D>::FLOATS;
+    float m = neg_inf(), l = 0.0f;
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c0 = 0; c0 < a.pf_split; c0 += kU) {
+        float mc[kU], lc[kU];
+        f32x4 oc[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const float* p = slot + (int64_t)min(c0 + u, a.pf_split - 1) * PrefillSlot<D>::FLOATS;
+            mc[u] = p[PrefillSlot<D>::M + rw];
+            lc[u] = p[PrefillSlot<D>::L + rw];
+            oc[u] = *reinterpret_cast<const f32x4*>(p + rw * D + d);
+        }
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            if (c0 + u >= a.pf_split) break;
+            const float mn = fmaxf(m, mc[u]);
+            // (equal references, both -inf among them, keep their sums as they are)
+            const float wo = m == mn ? 1.0f : fast_exp2(m - mn), wn = mc[u] == mn ? 1.0f : fast_exp2(mc[u] - mn);
+            l = l * wo + lc[u] * wn;
+            o = o * wo + oc[u] * wn;
+            m = mn;
+        }
+    }
+    const int jw = r / a.G, hd = g * a.G + r % a.G;
+    const float inv = l == 0.0f ? 0.0f : 1.0f / l;
+    st16(a.out + (int64_t)jw * a.o_nb2 + (int64_t)hd * a.o_nb1 + (int64_t)s * a.o_nb3 + 4 * d,
+         gated(a, o * inv, gate_load(a, s, jw, hd, d)));
 }
 
 template <int MODE, int D>
@@ -751,7 +829,7 @@ __global__ __launch_bounds__(kThreads, PfDim<D>::GROUPS) void prefill_gated(FaAr
 
 template <int MODE, int D, int KV>
 void launch_prefill_mode(const FaArgs& a, int causal, int nrb, hipStream_t stream) {
-    const dim3 grid((unsigned)((int64_t)a.S * a.H * nrb)), block(kThreads);
+    const dim3 grid((unsigned)((int64_t)a.S * a.Hkv * nrb * a.pf_split)), block(kThreads);
     if constexpr (KV == SIXI_TYPE_Q8_0)
         hipLaunchKernelGGL((prefill_q8<MODE, D>), grid, block, 0, stream, a, causal, nrb, a.P);
     else if (a.q_q8)
@@ -762,7 +840,7 @@ void launch_prefill_mode(const FaArgs& a, int causal, int nrb, hipStream_t strea
 
 template <int D, int KV, bool QQ8>
 void launch_gated(const FaArgs& a, int nrb, hipStream_t stream) {
-    const dim3 grid((unsigned)((int64_t)a.S * a.H * nrb)), block(kThreads);
+    const dim3 grid((unsigned)((int64_t)a.S * a.Hkv * nrb * a.pf_split)), block(kThreads);
     if constexpr (PfDim<D>::GROUPS == 1) {
         hipLaunchKernelGGL((prefill_gated<D, KV, QQ8, 0>), grid, block, 0, stream, a, nrb, a.P);
     } else {
@@ -787,7 +865,7 @@ template <int D, int KV>
 hipError_t launch_prefill_d(const FaArgs& a, int mask_mode, hipStream_t stream) {
     const bool generic = mask_mode == SIXI_MASK_EXPLICIT || a.softcap != 0.0f;
     const int causal = mask_mode == SIXI_MASK_BLOCK_CAUSAL;
-    const int nrb = (a.n_q + kBM - 1) / kBM;
+    const int nrb = prefill_row_blocks(a.n_q, a.G);
     // an explicit mask alone, with 16-byte aligned rows that one 32-bit range covers: LDS-staged
     const bool mask_only = mask_mode == SIXI_MASK_EXPLICIT && a.mask && a.softcap == 0.0f && a.alibi_nlog2 == 0 &&
                            reinterpret_cast<uintptr_t>(a.mask) % 16 == 0 && a.m_nb1 % 16 == 0 &&
@@ -800,7 +878,36 @@ hipError_t launch_prefill_d(const FaArgs& a, int mask_mode, hipStream_t stream) 
         launch_prefill_mode<MODE_GENERIC, D, KV>(a, causal, nrb, stream);
     else
         launch_prefill_mode<MODE_FAST, D, KV>(a, causal, nrb, stream);
+    if (a.pf_split > 1) {
+        const unsigned blocks = (unsigned)((int64_t)a.S * a.Hkv * nrb * (kBM / (kThreads / (D / 4))));
+        hipLaunchKernelGGL(prefill_merge<D>, dim3(blocks), dim3(kThreads), 0, stream, a);
+    }
     return hipGetLastError();
+}
+
+// Work-groups sharing each of `blocks` row blocks (1: no split).  Blocks that reach more than half
+// of the CUs are left whole: what idle CUs could take off them is then near what the sums' way
+// through memory costs.  A share walks n / C tiles and costs kStart tiles of start-up (Q, the
+// first tile, the sums' way out); its sums cross memory twice (kMerge tiles' time over the whole
+// chip).  Every C up to 16 whose launch stays within two full rounds is priced by its rounds; n_kv
+// stands in for the lengths, which only the device knows.
+int prefill_split(int64_t blocks, int64_t n_kv, int head_dim, int cu_count) {
+    if (2 * blocks > cu_count) return 1;
+    constexpr double kStart = 4.0;
+    const double kMerge = 0.05;
+    const int64_t slots = (int64_t)cu_count * prefill_groups_per_cu(head_dim);
+    const int64_t tiles = (n_kv + kPrefillCells - 1) / kPrefillCells;
+    int best = 1;
+    double best_cost = 0.0;
+    for (int c = 1; c <= 16 && (c == 1 || blocks * c <= 2 * slots) && (c == 1 || tiles >= 4 * c); ++c) {
+        const int64_t rounds = (blocks * c + slots - 1) / slots;
+        const double cost = (double)rounds * ((double)tiles / c + kStart) + (c > 1 ? kMerge * (double)(blocks * c) : 0.0);
+        if (c == 1 || cost < best_cost) {
+            best = c;
+            best_cost = cost;
+        }
+    }
+    return best;
 }
 
 hipError_t launch_prefill(const FaArgs& a, int kv_type, int mask_mode, int head_dim, hipStream_t stream) {

@@ -77,7 +77,23 @@ struct Plan {
     bool mask_prepass = false; // explicit mask reduced to per-row offsets first (fa_mask.hip)
     size_t prepass_offset = 0; // byte offset of its table (S * n_q int32), after the rest
     size_t ws_bytes = 0;
+    size_t ws_min = 0;         // the least a call can run with (ws_bytes without the prefill split)
+    size_t part_offset = 0;    // prefill split: byte offset of its sums (after the staging area)
 };
+
+// Prefill workspace: the staging area (or a token, so that the contract is uniform), the pre-pass
+// table, then the sums of `split` work-groups per row block.
+void prepass_layout(Plan& pl);
+void prefill_layout(Plan& pl, int split) {
+    pl.a.pf_split = split;
+    pl.ws_bytes = pl.stage_bytes > 0 ? pl.stage_bytes : kWsAlign;
+    prepass_layout(pl);
+    pl.ws_min = pl.ws_bytes;
+    if (split <= 1) return;
+    const int64_t blocks = (int64_t)pl.a.S * pl.a.Hkv * sixi::prefill_row_blocks(pl.a.n_q, pl.a.G);
+    pl.part_offset = align_up(pl.ws_bytes, kWsAlign);
+    pl.ws_bytes = pl.part_offset + align_up((size_t)(blocks * split * sixi::prefill_slot_floats(pl.D)) * sizeof(float), kWsAlign);
+}
 
 // Appends the pre-pass table to the workspace layout (after everything else, so that the
 // staging and split-K offsets do not move).
@@ -85,6 +101,11 @@ void prepass_layout(Plan& pl) {
     if (!pl.mask_prepass) return;
     pl.prepass_offset = align_up(pl.ws_bytes, kWsAlign);
     pl.ws_bytes = pl.prepass_offset + align_up((size_t)pl.a.S * pl.a.n_q * sizeof(int32_t), kWsAlign);
+}
+
+// Fewer shares per row block until the workspace fits in `bytes` (down to none).
+void prefill_fit(Plan& pl, size_t bytes) {
+    while (!pl.splitk && pl.a.pf_split > 1 && pl.ws_bytes > bytes) prefill_layout(pl, pl.a.pf_split - 1);
 }
 
 int cu_count_cached() {
@@ -354,11 +375,14 @@ int resolve(const sixi_attn_params* p, Plan* out, size_t stage_cap = SIXI_ATTN_S
         // slot indices run up to S*Hkv + P - 2 for a launch of P <= kMaxSplitGroups work-groups
         splitk_layout(pl, S * Hkv + sixi::kMaxSplitGroups);
     } else {
-        // the prefill kernel keeps everything on chip; a token workspace keeps the contract uniform
         if (S * H * ((n_q + 127) / 128) > (int64_t)INT32_MAX) return SIXI_E_UNSUPPORTED;
-        pl.ws_bytes = pl.stage_bytes > 0 ? pl.stage_bytes : kWsAlign;
+        const int64_t blocks = S * Hkv * sixi::prefill_row_blocks(n_q, a.G);
+        prefill_layout(pl, sixi::prefill_split(blocks, n_kv, pl.D, cu_count_cached()));
     }
-    prepass_layout(pl);
+    if (pl.splitk) {
+        prepass_layout(pl);
+        pl.ws_min = pl.ws_bytes;
+    }
     *out = pl;
     return SIXI_OK;
 }
@@ -396,6 +420,7 @@ int launch_groups(const Plan& pl) {
 
 // Launches a resolved call on `ws` (laid out as pl says).
 int run(Plan& pl, char* ws, hipStream_t stream) {
+    char* const ws0 = ws;
     FaArgs& a = pl.a;
     hipError_t e;
     if (pl.q8_stage) {
@@ -426,7 +451,7 @@ int run(Plan& pl, char* ws, hipStream_t stream) {
         if (sixi::launch_mask_prefix(a, stream) != hipSuccess) return SIXI_E_BACKEND;
     }
     if (pl.q8_stage) ws += pl.stage_bytes;
-    a.part = reinterpret_cast<float*>(ws);
+    a.part = reinterpret_cast<float*>(pl.splitk ? ws : ws0 + pl.part_offset);
     a.seg_pieces = pl.splitk ? reinterpret_cast<int32_t*>(ws + pl.seg_offset) : nullptr;
     a.P = launch_groups(pl);
 
@@ -462,11 +487,22 @@ int sixi_attn_workspace_bytes(const sixi_attn_params* p, size_t* bytes) {
     return SIXI_OK;
 }
 
+int sixi_attn_workspace_range(const sixi_attn_params* p, size_t* least, size_t* bytes) {
+    if (!least || !bytes) return SIXI_E_INVALID_ARGUMENT;
+    Plan pl;
+    const int rc = resolve(p, &pl);
+    if (rc != SIXI_OK) return rc;
+    *least = pl.ws_min;
+    *bytes = pl.ws_bytes;
+    return SIXI_OK;
+}
+
 int sixi_attn_forward(const sixi_attn_params* p) {
     Plan pl;
     int rc = resolve(p, &pl);
     if (rc != SIXI_OK) return rc;
-    if (!p->workspace || p->workspace_bytes < pl.ws_bytes) return SIXI_E_OUT_OF_BOUNDS;
+    if (!p->workspace || p->workspace_bytes < pl.ws_min) return SIXI_E_OUT_OF_BOUNDS;
+    prefill_fit(pl, p->workspace_bytes);
     if (!aligned(p->workspace, kWsAlign)) return SIXI_E_ALIGNMENT;
     // the kernels write the workspace while they read the views
     if (workspace_overlaps(p, p->workspace, pl.ws_bytes)) return SIXI_E_INVALID_ARGUMENT;
@@ -483,6 +519,7 @@ int sixi_attn_forward_noalloc(const sixi_attn_params* p) {
         splitk_layout(pl, (int64_t)pl.a.S * pl.a.Hkv + launch_groups(pl));
         prepass_layout(pl);
     }
+    prefill_fit(pl, kScratchBytes);
     if (pl.ws_bytes > kScratchBytes) return SIXI_E_OUT_OF_BOUNDS;
     char* base = scratch_base();
     if (!base) return SIXI_E_BACKEND;

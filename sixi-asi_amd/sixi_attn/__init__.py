@@ -44,6 +44,7 @@ EXPORTED_SYMBOLS = (
     "sixi_attn_forward",
     "sixi_attn_forward_noalloc",
     "sixi_attn_workspace_bytes",
+    "sixi_attn_workspace_range",
     "sixi_attn_validate",
     "sixi_attn_strerror",
     "sixi_attn_abi_version",
@@ -225,6 +226,8 @@ def load_library(path: Optional[os.PathLike] = None) -> ctypes.CDLL:
     lib.sixi_attn_validate.restype = ctypes.c_int
     lib.sixi_attn_workspace_bytes.argtypes = [P, ctypes.POINTER(ctypes.c_size_t)]
     lib.sixi_attn_workspace_bytes.restype = ctypes.c_int
+    lib.sixi_attn_workspace_range.argtypes = [P, ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)]
+    lib.sixi_attn_workspace_range.restype = ctypes.c_int
     lib.sixi_attn_strerror.argtypes = [ctypes.c_int]
     lib.sixi_attn_strerror.restype = ctypes.c_char_p
     lib.sixi_attn_abi_version.argtypes = []
@@ -311,7 +314,9 @@ def view_of(t, type_id: Optional[int] = None, head_dim: Optional[int] = None,
 class FlashAttnExt:
     """``ggml_flash_attn_ext`` over per-stream KV caches on one gfx950 GPU.
 
-    Keeps a device workspace (grown on demand) so repeated calls allocate nothing.  A buffer
+    Keeps a device workspace (grown on demand) so repeated calls allocate nothing; prefill calls that
+    split their row blocks over idle CUs keep one per stream beside it, so that a prefill may overlap
+    calls on other streams (under capture, or with an explicit ``stream``, they run unsplit).  A buffer
     that a larger call supersedes stays allocated for the life of the object, so a HIP graph
     captured over an earlier call still owns the memory its kernels write.  A caller may
     also pass its own ``workspace`` (a uint8 device tensor of at least
@@ -324,6 +329,7 @@ class FlashAttnExt:
         self.lib = load_library()
         self.device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
         self._ws = None
+        self._split_ws = {}  # stream -> workspace of the prefill calls that split their row blocks
         self._retired = []  # superseded workspaces: graphs captured before a regrowth still use them
 
     def params(self, q, k, v, out, kv_len=None, q_len=None, mask_mode=MASK_BLOCK_CAUSAL, mask=None,
@@ -378,6 +384,15 @@ class FlashAttnExt:
             self._ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=self.device)
         return self._ws
 
+    def _split_workspace(self, stream: int, nbytes: int):
+        import torch
+
+        ws = self._split_ws.get(stream)
+        if ws is None or ws.numel() < nbytes:
+            # (a superseded buffer goes back to the allocator, whose next use of it this stream orders)
+            ws = self._split_ws[stream] = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        return ws
+
     def __call__(self, q, k, v, out, kv_len=None, q_len=None, mask_mode=MASK_BLOCK_CAUSAL, mask=None,
                  scale=None, max_bias=0.0, logit_softcap=0.0, kv_type=None, stream=None, check=True,
                  workspace=None, noalloc=False, page_table=None, bounded_workspace=False, gate=None) -> int:
@@ -396,12 +411,20 @@ class FlashAttnExt:
             if check and rc != OK:
                 raise SixiAttnError(rc, strerror(rc))
             return rc
-        n = ctypes.c_size_t(0)
-        rc = self.lib.sixi_attn_workspace_bytes(ctypes.byref(p), ctypes.byref(n))
+        least, n = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        rc = self.lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(n))
         if rc == OK:
-            ws = self._workspace(n.value) if workspace is None else workspace
+            size = None
+            if workspace is not None:
+                ws = workspace
+            elif least.value == n.value:
+                ws = self._workspace(n.value)
+            elif stream is None and not torch.cuda.is_current_stream_capturing():
+                ws = self._split_workspace(p.stream, n.value)
+            else:
+                ws, size = self._workspace(least.value), least.value
             p.workspace = ws.data_ptr()
-            p.workspace_bytes = ws.numel() * ws.element_size()
+            p.workspace_bytes = ws.numel() * ws.element_size() if size is None else size
             rc = self.lib.sixi_attn_forward(ctypes.byref(p))
         if check and rc != OK:
             raise SixiAttnError(rc, strerror(rc))

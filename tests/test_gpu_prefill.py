@@ -155,3 +155,56 @@ def test_prefill_f16_queries(fa):
     want = oracle.attention_for_workload(ref_host, w.kv_type)
     for s in range(w.S):
         _check(want[s, :w.q_len[s]], got[s, :w.q_len[s]], f"f16 Q stream {s}")
+
+
+@pytest.mark.parametrize("kv_len,q_len,H,Hkv,D,kv,mode", [
+    ([1500], [17], 24, 4, 128, sa.TYPE_F16, "lengths"),         # 102 rows: one row block, 6 of them empty
+    ([700, 0, 5], [22, 17, 0], 24, 4, 256, sa.TYPE_F16, "lengths"),  # a second block of 4 rows; shares with no cell
+    ([4100], [65], 8, 2, 128, sa.TYPE_Q8_0, "lengths"),         # three blocks, 66 tiles, q8_0
+    ([3000, 900], [33, 20], 24, 4, 256, sa.TYPE_Q8_0, "lengths"),
+    ([2000, 30], [40, 31], 24, 4, 128, sa.TYPE_F16, "causal"),    # the causal mask, handed over
+    ([2000, 30], [40, 31], 24, 4, 256, sa.TYPE_F16, "holes"),     # a mask with holes: the staged-mask body
+    ([1100], [24], 24, 4, 128, sa.TYPE_F16, "softcap"),          # the per-cell body
+])
+def test_split_row_blocks(fa, kv_len, q_len, H, Hkv, D, kv, mode):
+    """Few row blocks over a long cache: several work-groups share the cells of each.  Against the
+    oracle (the bar above), and against the same call with the least workspace (no split): the two
+    differ by the order of f32 sums and the exponent references the f16 probabilities were taken
+    against, 2^-11 of rounding each, averaged over the cells: a tenth of the bar's rel-L2 more."""
+    import ctypes
+
+    _say(f"split kv_len={kv_len} q_len={q_len} H={H} Hkv={Hkv} D={D} kv={kv} {mode}")
+    w = wl.Workload("split_prefill", 0x51A7_5100 + sum(q_len) + D, len(kv_len), kv_len, q_len, H=H, Hkv=Hkv, D=D, kv_type=kv)
+    host = wl.make_host(w, poison=True)
+    dev = wl.to_device(host)
+    kw = dict(kv_len=dev["kv_len"], q_len=dev["q_len"])
+    n_kv = dev["k"].shape[1]
+    if mode in ("causal", "holes"):
+        last = torch.tensor(kv_len)[:, None, None] + torch.arange(w.n_q)[None, :, None]
+        seen = torch.arange(n_kv)[None, None] <= last
+        if mode == "holes":
+            seen &= (torch.arange(n_kv) % 7 != 3)[None, None]
+        mask = torch.where(seen, 0.0, float("-inf")).to(torch.float16)[:, None].contiguous().cuda()
+        kw.update(mask_mode=sa.MASK_EXPLICIT, mask=mask)
+    if mode == "softcap":
+        kw.update(logit_softcap=20.0)
+    outs = []
+    for split in (True, False):
+        out = torch.full((w.S, w.n_q, w.H, w.D), float("nan"), dtype=torch.float32, device="cuda")
+        p = fa.params(dev["q"], dev["k"], dev["v"], out, **kw)
+        least, full = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert fa.lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(full)) == sa.OK
+        assert least.value < full.value, "the case is meant to split"
+        ws = torch.full((full.value if split else least.value,), 0xFF, dtype=torch.uint8, device="cuda")
+        fa(dev["q"], dev["k"], dev["v"], out, workspace=ws, **kw)
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+    got, whole = (np.concatenate([o[s, :q_len[s]].ravel() for s in range(w.S)]) for o in outs)
+    for s in range(w.S):  # rows past q_len are not written
+        assert np.all(np.isnan(outs[0][s, q_len[s]:]))
+    m = oracle.diff_metrics(whole, got)
+    _say(f"split against whole: rel_l2={m['rel_l2']:.3e}")
+    assert m["rel_l2"] <= 1.1 * REL_L2, m
+    if mode in ("lengths", "causal"):
+        want = oracle.attention_for_workload(host, w.kv_type)
+        _check(np.concatenate([want[s, :q_len[s]].ravel() for s in range(w.S)]), got, "split")
