@@ -7,7 +7,7 @@
 //   delta = beta * (v[h] - sk);   S[h][s] = alpha S[h][s] + delta k[s];   y[h] = sum_s S[h][s] q[s]
 // The reference runs one launch per token and stream with the state in HBM; here the state of a
 // (stream, group) is read once and written once (at the snapshot row), and a block of rows runs on
-// chip.  Two kernels:
+// chip.  Three kernels:
 //
 // gdn_verify_chunked_kernel (128-dim keys, states of 128 or 64 rows: the model's linear-attention
 // layers hold 128 x 128) runs 16 rows at a time in the closed ("WY") form of the delta rule, on the f32 matrix
@@ -17,6 +17,10 @@
 // against 64-65 us for the step by step kernel below; launching one item per work-group it
 // measured 63.7 us (every work-group of a CU then loads, computes and stores in step), and without
 // the XCD pairing of the two halves of a state 60.5 us.
+//
+// gdn_scan_kernel (the same shapes, while the work-groups fit the CUs at once: a prompt chunk, or a
+// short block of one or a few streams) runs the chunks of a state as a pipeline; its comment has
+// the split.
 //
 // gdn_verify_kernel (64-dim keys) steps token by token on the VALU with the state in registers;
 // the decay alpha goes into a scalar factor of the carried state (S = cs * st, below), not into
@@ -507,6 +511,334 @@ __global__ __launch_bounds__(256) void gdn_verify_chunked_kernel(GdnArgs a, int 
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Long blocks of few streams (a prompt chunk): the chunks of a state are a serial chain, and one
+// chain per 64 state rows leaves most of the chip idle.  The chunked kernel above spends 5.8 us per
+// chunk there (one stream, 48 groups, 2048 rows: 741 us), of which the matrix cores need 1.6: each
+// chunk's loads, Gram products, triangular inverse and state products run one after another.
+//
+// Here a work-group of eight waves owns 32 state rows (HD / 32 work-groups per state) and runs the
+// same algebra as a pipeline over the chunks, an iteration in two halves with a barrier after each:
+//   waves 0..3 (consumers) take chunk i: wave = 16 state rows x 64 columns, so P = S0 k^T and
+//     Z = S0 q^T are half sums, exchanged through LDS between the halves; then U, y and the state's
+//     update, whose operands were read in the first half;
+//   waves 4..7 (producers) prepare what does not depend on the state.  Second half: waves 4, 5 hold
+//     k (64 columns each) of chunk i + 3 in registers, put it into LDS and sum k k^T, waves 6, 7
+//     the same with q and k q^T.  First half: wave 4 makes L and wave 6 makes W of chunk i + 2,
+//     wave 7 stages v, the gates and their products E of chunk i + 3, wave 5 inverts I + L of chunk
+//     i + 1.  Each issues the global loads of its chunk two iterations ahead.
+// Every SIMD holds one consumer and one producer, whose 56 and 16 f32 MFMAs (32 cycles each) per
+// iteration are its floor: 2304 cycles, 123 us over the 128 chunks of 2048 rows, which take 325 us:
+// the producers switched off leave 219 (the consumers' chain P -> exchange -> U -> state), the
+// inversion alone is 35 of it, the staging loads 28, E 27, k k^T and k q^T 24.
+constexpr int kScanRows = 32;
+
+struct GdnScanLds {
+    float k[3][kCT][kCP], q[3][kCT][kCP];  // chunk c at c % 3
+    float v[4][kCT][kScanRows];            // chunk c at c % 4 (E, A, C, B, W alike)
+    float E[4][kCT][kCT];                  // E[t][s], 0 for s > t
+    float A[4][kCT], C[4][kCT], B[4][kCT]; // A_t, c_t, beta_t
+    float W[4][kCT][kCT];                  // W[t][s] = E[t][s] (k_s . q_t)
+    float L[2][kCT][kCT], M[2][kCT][kCT];  // chunk c at c % 2; M = (I + L)^-1
+    f32x4 P[4][64], Z[2][64];              // half sums of the consumers (Z: of the upper columns)
+    f32x4 G[2][64];                        // half sums of the Gram products (upper columns)
+};
+
+// Work-group barrier for LDS traffic: global loads stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <int HD, bool DECAY_FIRST>
+__global__ __launch_bounds__(512) void gdn_scan_kernel(GdnArgs a, int grouped) {
+    constexpr int K = 128, T = kCT, SPLIT = HD / kScanRows;
+    static_assert(HD % kScanRows == 0 && K == 2 * 64, "two column halves");
+    __shared__ __align__(16) GdnScanLds sh;
+
+    // the work-groups of one state read the same q and k: with `grouped` (states a multiple of 8)
+    // they are dealt to one XCD
+    const int b = blockIdx.x;
+    const int state = grouped ? (b >> 3) / SPLIT * 8 + (b & 7) : b / SPLIT;
+    const int hr0 = ((grouped ? b >> 3 : b) % SPLIT) * kScanRows;
+    const int g = state % a.G, s = state / a.G;
+    int ql = a.q_len ? a.q_len[s] : a.n_rows;
+    ql = ql < 0 ? 0 : (ql > a.n_rows ? a.n_rows : ql);
+    int snap = a.snap ? a.snap[s] : ql;
+    snap = snap < 0 ? 0 : (snap > ql ? ql : snap);
+    const int n_chunks = (ql + T - 1) / T;
+
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, lr = lane & 15, gl = lane >> 4;
+
+    if (wv < 4) {
+        const int kh = wv & 1;                    // column half
+        const int hw = 16 * (wv >> 1) + lr;       // the lane's state row in the work-group
+        const int h = hr0 + hw;
+        const int64_t col = 256 * kh + 16 * gl;   // bytes
+        const char* const sin = a.s_in + (int64_t)g * a.si_nb2 + (int64_t)s * a.si_nb3 + (int64_t)h * a.si_nb1 + col;
+        char* const sout = a.s_out + (int64_t)g * a.so_nb2 + (int64_t)s * a.so_nb3 + (int64_t)h * a.so_nb1 + col;
+        f32x4 st[4];  // columns 64 kh + 16 m + 4 gl + j in st[m][j]
+#pragma unroll
+        for (int m = 0; m < 4; ++m) st[m] = *reinterpret_cast<const f32x4*>(sin + 64 * m);
+        if (snap == 0) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) *reinterpret_cast<f32x4*>(sout + 64 * m) = st[m];
+        }
+        char* const yb = a.y + (int64_t)g * a.y_nb1 + (int64_t)s * a.y_nb3 + (int64_t)h * 4;
+        // rows lr of k and q of the chunk ahead, as P's and Z's A operands
+        f32x4 kx[4], qx[4];
+        auto read_rows = [&](int c) {
+            const int b3 = c % 3;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                kx[m] = *reinterpret_cast<const f32x4*>(&sh.k[b3][lr][64 * kh + 16 * m + 4 * gl]);
+                qx[m] = *reinterpret_cast<const f32x4*>(&sh.q[b3][lr][64 * kh + 16 * m + 4 * gl]);
+            }
+        };
+        for (int i = -3; i < 0; ++i) {
+            lds_barrier();
+            if (i == -1 && n_chunks > 0) read_rows(0);
+            lds_barrier();
+        }
+        for (int i = 0; i < n_chunks; ++i) {
+            const int b3 = i % 3, b4 = i & 3;
+            const int t0 = i * T, nt = ql - t0 < T ? ql - t0 : T;
+            const bool more = t0 + T < ql;
+            const bool snap_here = snap > t0 && snap <= t0 + nt;
+            // what the second half needs of the producers' work
+            float ka[4][4], vv[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                vv[j] = sh.v[b4][4 * gl + j][hw];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) ka[m][j] = sh.k[b3][4 * gl + j][64 * kh + 16 * m + lr];
+            }
+            const f32x4 mx = *reinterpret_cast<const f32x4*>(&sh.M[i & 1][lr][4 * gl]);
+            const f32x4 wx = *reinterpret_cast<const f32x4*>(&sh.W[b4][lr][4 * gl]);
+            const f32x4 ax = *reinterpret_cast<const f32x4*>(&sh.A[b4][4 * gl]);
+            const f32x4 cx = *reinterpret_cast<const f32x4*>(&sh.C[b4][4 * gl]);
+            const f32x4 bx = *reinterpret_cast<const f32x4*>(&sh.B[b4][4 * gl]);
+            const f32x4 el = *reinterpret_cast<const f32x4*>(&sh.E[b4][T - 1][4 * gl]);
+            const float al = sh.A[b4][T - 1];
+            f32x4 pt[2], zt[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) pt[u] = zt[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    pt[m & 1] = mma4(kx[m][j], st[m][j], pt[m & 1]);
+                    zt[m & 1] = mma4(qx[m][j], st[m][j], zt[m & 1]);
+                }
+            f32x4 p = pt[0] + pt[1];
+            const f32x4 z = zt[0] + zt[1];
+            sh.P[wv][lane] = p;
+            if (kh) sh.Z[wv >> 1][lane] = z;
+            lds_barrier();
+            p += sh.P[wv ^ 1][lane];
+            const f32x4 zp = sh.Z[wv >> 1][lane];
+            if (more) read_rows(i + 1);
+            // U^T = M R^T (lane: U[h][4 gl + j] in register j)
+            f32x4 ut = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ut = mma4(mx[j], bx[j] * (vv[j] - cx[j] * p[j]), ut);
+            if (snap_here) {
+                // S_sigma = A_sigma S0 + k^T (U E[sigma])^T, to the output state
+                const int sig = snap - 1 - t0;
+                const float as = sh.A[b4][sig];
+                const f32x4 ub = ut * *reinterpret_cast<const f32x4*>(&sh.E[b4][sig][4 * gl]);
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    f32x4 acc = st[m] * as;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc = mma4(ka[m][j], ub[j], acc);
+                    *reinterpret_cast<f32x4*>(sout + 64 * m) = acc;
+                }
+            }
+            // the next chunk's S0 (sigma = T - 1; unused after the last chunk) and, between its
+            // MFMAs, y^T = diag(A) Z^T + W^T U^T (kept by the lower columns' wave)
+            const f32x4 ub = ut * el;
+            f32x4 yt = ax * (z + zp);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) st[m] *= al;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) st[m] = mma4(ka[m][j], ub[j], st[m]);
+                yt = mma4(wx[j], ut[j], yt);
+            }
+            if (!kh) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (4 * gl + j < nt) *reinterpret_cast<float*>(yb + (int64_t)(t0 + 4 * gl + j) * a.y_nb2) = yt[j];
+            }
+            lds_barrier();
+        }
+        return;
+    }
+
+    // ---- producers ----
+    const int pw = wv - 4;
+    const int half = pw & 1;
+    const bool is_q = pw >= 2;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const char* const kb = a.k + (int64_t)g * a.k_nb1 + (int64_t)s * a.k_nb3 + 256 * half + 16 * gl;
+    const char* const qb = a.q + (int64_t)g * a.q_nb1 + (int64_t)s * a.q_nb3 + 256 * half + 16 * gl;
+    // a chunk in registers: row lr, columns 64 half + 16 m + 4 gl .. + 3 (zeros past the block); in
+    // wave 7 also the gates of row lr (1 and 0 past the block) and rows lane / 8, 8 + lane / 8 of v
+    struct Chunk {
+        f32x4 k[4], q[4], v[2];
+        float al, be;
+    };
+    auto load_rows = [&](int c, Chunk& x) {
+        const int t = c * T + lr;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) x.k[m] = x.q[m] = zero;
+        if (t < ql) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                x.k[m] = *reinterpret_cast<const f32x4*>(kb + (int64_t)t * a.k_nb2 + 64 * m);
+                if (is_q) x.q[m] = *reinterpret_cast<const f32x4*>(qb + (int64_t)t * a.q_nb2 + 64 * m);
+            }
+        }
+    };
+    auto load_gates = [&](int c, Chunk& x) {
+        const int t = c * T + lr;
+        x.al = 1.0f;
+        x.be = 0.0f;
+        if (t < ql) {
+            x.al = *reinterpret_cast<const float*>(a.alpha + (int64_t)g * a.a_nb0 + (int64_t)t * a.a_nb1 + (int64_t)s * a.a_nb2);
+            x.be = *reinterpret_cast<const float*>(a.beta + (int64_t)g * a.b_nb0 + (int64_t)t * a.b_nb1 + (int64_t)s * a.b_nb2);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int tv = c * T + 8 * u + (lane >> 3);
+            x.v[u] = zero;
+            if (tv < ql)
+                x.v[u] = *reinterpret_cast<const f32x4*>(a.v + (int64_t)g * a.v_nb1 + (int64_t)tv * a.v_nb2 +
+                                                         (int64_t)s * a.v_nb3 + 4 * hr0 + 16 * (lane & 7));
+        }
+    };
+    // M = (I + L)^-1 by blocks: the 4 x 4 diagonal blocks in closed form (D), then twice
+    // M <- M - M Lo M with Lo the blocks below the diagonal of the doubled blocks, on the matrix
+    // cores (elimination row by row in one wave took 0.6 us of a 2.8 us iteration).  A product's
+    // accumulator layout is its B operand's: lane = column lr, rows 4 gl + j.
+    auto invert = [&](float (&L)[T][T], float (&M)[T][T]) {
+        const int bk = lr >> 2, p = lr & 3;
+        const f32x4 l1 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 1][4 * bk]);
+        const f32x4 l2 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 2][4 * bk]);
+        const f32x4 l3 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 3][4 * bk]);
+        const f32x4 lx = *reinterpret_cast<const f32x4*>(&L[lr][4 * gl]);
+        const float m10 = -l1[0], m21 = -l2[1], m32 = -l3[2];
+        const float m20 = -fmaf(l2[1], m10, l2[0]), m31 = -fmaf(l3[2], m21, l3[1]);
+        const float m30 = -fmaf(l3[2], m20, fmaf(l3[1], m10, l3[0]));
+        const bool diag = gl == bk;
+        f32x4 row = p == 0 ? f32x4{1.0f, 0.0f, 0.0f, 0.0f} : p == 1 ? f32x4{m10, 1.0f, 0.0f, 0.0f}
+                  : p == 2 ? f32x4{m20, m21, 1.0f, 0.0f} : f32x4{m30, m31, m32, 1.0f};
+        f32x4 col = p == 0 ? f32x4{1.0f, m10, m20, m30} : p == 1 ? f32x4{0.0f, 1.0f, m21, m31}
+                  : p == 2 ? f32x4{0.0f, 0.0f, 1.0f, m32} : f32x4{0.0f, 0.0f, 0.0f, 1.0f};
+        row = diag ? row : zero;  // D[lr][4 gl + j]
+        col = diag ? col : zero;  // D[4 gl + j][lr]
+        const f32x4 lo4 = gl + 1 == bk && (bk & 1) ? lx : zero;
+        const f32x4 lo8 = gl < 2 && bk >= 2 ? lx : zero;
+        f32x4 x = zero, m8 = col;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x = mma4(lo4[j], col[j], x);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m8 = mma4(-row[j], x[j], m8);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) M[4 * gl + j][lr] = m8[j];
+        x = zero;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x = mma4(lo8[j], m8[j], x);
+        const f32x4 mrow = *reinterpret_cast<const f32x4*>(&M[lr][4 * gl]);
+        f32x4 m16 = m8;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m16 = mma4(-mrow[j], x[j], m16);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) M[4 * gl + j][lr] = m16[j];
+    };
+    f32x4 gr = zero;  // this wave's Gram product of chunk i + 2, then of chunk i + 3
+    // iteration i; x holds chunk i + 3 and takes chunk i + 5
+    auto iteration = [&](int i, Chunk& x) {
+        if (half == 0 && i + 2 >= 0 && i + 2 < n_chunks) {
+            const int b4 = (i + 2) & 3, b2 = i & 1;
+            gr += sh.G[is_q][lane];  // k_{4gl+r} . k_lr (or . q_lr)
+            if (is_q) {
+                const f32x4 ex = *reinterpret_cast<const f32x4*>(&sh.E[b4][lr][4 * gl]);
+                *reinterpret_cast<f32x4*>(&sh.W[b4][lr][4 * gl]) = ex * gr;  // 0 past the diagonal
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = 4 * gl + r;
+                    float l = 0.0f;
+                    if (lr < t) l = sh.B[b4][t] * (DECAY_FIRST ? sh.E[b4][t][lr] : sh.E[b4][t - 1][lr]) * gr[r];
+                    sh.L[b2][t][lr] = l;
+                }
+            }
+        }
+        if (pw == 1 && i + 1 >= 0 && i + 1 < n_chunks) invert(sh.L[(i + 1) & 1], sh.M[(i + 1) & 1]);
+        const bool on = i + 3 < n_chunks;
+        if (pw == 3 && on) {
+            const int b4 = (i + 3) & 3;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) *reinterpret_cast<f32x4*>(&sh.v[b4][8 * u + (lane >> 3)][4 * (lane & 7)]) = x.v[u];
+            // column lr of E, multiplied in row order; this lane's rows 4 gl .. + 3
+            float e = 1.0f, ev[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            const int ai = __builtin_bit_cast(int, x.al);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const float at = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, t));
+                if (t > lr) e *= at;
+                if (gl == t / 4) ev[t % 4] = t >= lr ? e : 0.0f;
+            }
+            const float a0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, 0));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int t = 4 * gl + r;
+                sh.E[b4][t][lr] = ev[r];
+                if (lr == 0) {
+                    sh.A[b4][t] = ev[r] * a0;
+                    if (DECAY_FIRST) sh.C[b4][t] = ev[r] * a0;
+                    else if (t + 1 < T) sh.C[b4][t + 1] = ev[r] * a0;
+                }
+            }
+            if (!DECAY_FIRST && lane == 0) sh.C[b4][0] = 1.0f;
+            if (gl == 0) sh.B[b4][lr] = x.be;
+            if (i + 5 < n_chunks) load_gates(i + 5, x);
+        }
+        lds_barrier();
+        if (on) {
+            const int b3 = (i + 3) % 3;
+            f32x4 g2[2] = {zero, zero};
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                *reinterpret_cast<f32x4*>(is_q ? &sh.q[b3][lr][64 * half + 16 * m + 4 * gl]
+                                               : &sh.k[b3][lr][64 * half + 16 * m + 4 * gl]) = is_q ? x.q[m] : x.k[m];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) g2[m & 1] = mma4(x.k[m][j], is_q ? x.q[m][j] : x.k[m][j], g2[m & 1]);
+            }
+            gr = g2[0] + g2[1];
+            if (half) sh.G[is_q][lane] = gr;
+            if (i + 5 < n_chunks) load_rows(i + 5, x);
+        }
+        lds_barrier();
+    };
+    Chunk even, odd;
+    load_rows(0, even);
+    load_rows(1, odd);
+    if (pw == 3) {
+        load_gates(0, even);
+        load_gates(1, odd);
+    }
+    for (int i = -3; i < n_chunks; i += 2) {
+        iteration(i, even);
+        if (i + 1 < n_chunks) iteration(i + 1, odd);
+    }
+}
+
 // Work-groups of the chunked kernel that fit the device at once (each then runs several items).
 template <int HD, bool DECAY_FIRST>
 int chunked_resident_groups() {
@@ -537,8 +869,34 @@ hipError_t launch_chunked_df(const GdnArgs& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+int cu_count() {
+    static int cached = -1;
+    if (cached < 0) {
+        int dev = 0, n = 0;
+        cached = hipGetDevice(&dev) == hipSuccess &&
+                 hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? n : 0;
+    }
+    return cached;
+}
+
+template <int HD>
+hipError_t launch_scan(const GdnArgs& a, hipStream_t stream) {
+    const int64_t groups = (int64_t)a.S * a.G * (HD / kScanRows);
+    const int grouped = ((int64_t)a.S * a.G) % 8 == 0;
+    if (a.decay_first)
+        hipLaunchKernelGGL((gdn_scan_kernel<HD, true>), dim3((unsigned)groups), dim3(512), 0, stream, a, grouped);
+    else
+        hipLaunchKernelGGL((gdn_scan_kernel<HD, false>), dim3((unsigned)groups), dim3(512), 0, stream, a, grouped);
+    return hipGetLastError();
+}
+
 template <int HD>
 hipError_t launch_chunked(const GdnArgs& a, hipStream_t stream) {
+    // While its work-groups fit the CUs at once the scan kernel is the faster one at every length (48
+    // groups, one stream: 4 rows 9.4 -> 8.7 us, 16 rows 9.6 -> 9.0, 33 rows 18.1 -> 15.0, 2048 rows
+    // 741 -> 337 with the launch); beyond that its eight waves per CU lose to the sixteen of the chunked kernel (two
+    // streams, an earlier form of it: 16 rows 10.1 against 15.0 us, 128 rows 46 against 55).
+    if ((int64_t)a.S * a.G * (HD / kScanRows) <= cu_count()) return launch_scan<HD>(a, stream);
     return a.decay_first ? launch_chunked_df<HD, true>(a, stream) : launch_chunked_df<HD, false>(a, stream);
 }
 
