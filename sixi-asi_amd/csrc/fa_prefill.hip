@@ -107,7 +107,9 @@ __device__ __forceinline__ f32x16 mfma32x32x16(f16x8 a, f16x8 b, f32x16 c) {
 
 // QQ8: Q goes through ggml's conversion to the q8_0 dot type (a q8_0 cache, read as q8_0 tiles or
 // staged as f16 rows).
-template <int MODE, int D, int KV, bool QQ8>
+// LEAN: the DMA offsets of the K/V tiles are worked out per tile instead of held in registers (256-dim
+// heads where a staged mask, or a mask body in the same kernel, leaves none for them).
+template <int MODE, int D, int KV, bool QQ8, bool LEAN = D == 256 && MODE == MODE_MASK>
 __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nrb, int n_cu,
                                              PrefillLds<D, MODE == MODE_MASK>& sh) {
     using P = PfDim<D>;
@@ -258,22 +260,28 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
     for (int ks = 0; ks < P::KS; ++ks) koff[ks] = rl * P::ROW + ((((2 * ks + hl) ^ (rl & 15)) & (P::CPR - 1)) << 4);
     // K staging: wave w's load u fills cells CPL(LW w + u) + l/CPR; lane fetches chunk (l%CPR)^cell
     // (the XOR touches the low four bits of the chunk index)
-    uint32_t kdo[P::LW];
+    auto k_offsets = [&](int l, uint32_t (&o)[P::LW]) {
 #pragma unroll
-    for (int u = 0; u < P::LW; ++u) {
-        const int cell = P::CPL * (P::LW * w + u) + lane / P::CPR;
-        kdo[u] = (uint32_t)cell * knb + (uint32_t)(((lane % P::CPR) ^ (cell & 15)) * 16);
-    }
+        for (int u = 0; u < P::LW; ++u) {
+            const int cell = P::CPL * (P::LW * w + u) + l / P::CPR;
+            o[u] = (uint32_t)cell * knb + (uint32_t)(((l % P::CPR) ^ (cell & 15)) * 16);
+        }
+    };
+    uint32_t kdo[P::LW];
+    if constexpr (!LEAN) k_offsets(lane, kdo);
     // V staging: wave w's load u fills LDS row CPL(LW w + u) + t/CPR at 16-byte position
     // t%CPR, i.e. 32-byte chunk position (t%CPR)/2 of the row, which holds dims
     // 16 * (position ^ 2(row % 4))
-    uint32_t vdo[P::LW];
+    auto v_offsets = [&](int l, uint32_t (&o)[P::LW]) {
 #pragma unroll
-    for (int u = 0; u < P::LW; ++u) {
-        const int cell = P::CPL * (P::LW * w + u) + lane / P::CPR;
-        const int pos = lane % P::CPR;
-        vdo[u] = (uint32_t)cell * vnb + 32u * (uint32_t)((pos >> 1) ^ (2 * (cell & 3))) + 16u * (uint32_t)(pos & 1);
-    }
+        for (int u = 0; u < P::LW; ++u) {
+            const int cell = P::CPL * (P::LW * w + u) + l / P::CPR;
+            const int pos = l % P::CPR;
+            o[u] = (uint32_t)cell * vnb + 32u * (uint32_t)((pos >> 1) ^ (2 * (cell & 3))) + 16u * (uint32_t)(pos & 1);
+        }
+    };
+    uint32_t vdo[P::LW];
+    if constexpr (!LEAN) v_offsets(lane, vdo);
     // V^T A operand of (db, kk), half h: lane (G = l/16, q = l%16) addresses cell
     // 16kk + 8h + x, x = 4(G/2) + q/4, dims 32db + 16(G%2) + 4(q%4) .. +3, which sits in chunk
     // position (2db + G%2) ^ 2(x % 4).  The row offset has the bits that 64db touches clear,
@@ -292,6 +300,10 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
         const int page = t * kBN < sd.nc ? page_id(pages, a, s, (t * kBN) >> 8) : 0;
         const KvSpan ksp = kv_span(a, a.k, a.k_nb1, a.k_nb2, a.k_nb3, s, g, t * kBN, sd.nc, rowb, page);
         const KvSpan vsp = kv_span(a, a.v, a.v_nb1, a.v_nb2, a.v_nb3, s, g, t * kBN, sd.nc, rowb, page);
+        if constexpr (LEAN) {
+            k_offsets(opaque(lane), kdo);
+            v_offsets(opaque(lane), vdo);
+        }
         const buf_rsrc krs = make_rsrc_uniform(ksp.p, ksp.bytes);
         const buf_rsrc vrs = make_rsrc_uniform(vsp.p, vsp.bytes);
         if constexpr (P::LW == 4) {
@@ -702,32 +714,29 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
     asm volatile("" : "+v"(lx));
     const int hw = lx >> 5;
     const int rw = 32 * wq + (lx & 31);  // row in the group
-    if (a.pf_split > 1) {
-        // a split item: this share's plain sums and their exponent reference (log2 units)
-        if (r0 + rw >= n_rows) return;
-        float* slot = a.part + (int64_t)(chunk + a.pf_split * (g + a.Hkv * (s + a.S * rb))) * PrefillSlot<D>::FLOATS;
-        char* dst = reinterpret_cast<char*>(slot + rw * D);
-#pragma unroll
-        for (int db = 0; db < P::DB; ++db)
-#pragma unroll
-            for (int bq = 0; bq < 4; ++bq)
-                st16(dst + (32 * db + 8 * bq + 4 * hw) * 4,
-                     f32x4{acc[db][4 * bq], acc[db][4 * bq + 1], acc[db][4 * bq + 2], acc[db][4 * bq + 3]});
-        if (hw == 0) {
-            slot[PrefillSlot<D>::M + rw] = RAW ? m_ref * c2 : m_ref;
-            slot[PrefillSlot<D>::L + rw] = l_sum;
-        }
-    } else if (r0 + rw < n_rows) {
+    if (r0 + rw < n_rows) {
+        const bool share = a.pf_split > 1;  // a split item's share: plain sums, and their exponent reference (log2 units)
         const int jw = (r0 + rw) / a.G, hd = g * a.G + (r0 + rw) % a.G;
-        const float inv = l_sum == 0.0f ? 0.0f : 1.0f / l_sum;
+        float inv = l_sum == 0.0f ? 0.0f : 1.0f / l_sum;
         char* dst = a.out + (int64_t)jw * a.o_nb2 + (int64_t)hd * a.o_nb1 + (int64_t)s * a.o_nb3;
+        if (share) {
+            float* slot = a.part + (int64_t)(chunk + a.pf_split * (g + a.Hkv * (s + a.S * rb))) * PrefillSlot<D>::FLOATS;
+            if (hw == 0) {
+                slot[PrefillSlot<D>::M + rw] = RAW ? m_ref * c2 : m_ref;
+                slot[PrefillSlot<D>::L + rw] = l_sum;
+            }
+            inv = 1.0f;
+            dst = reinterpret_cast<char*>(slot + rw * D);
+        }
 #pragma unroll
         for (int db = 0; db < P::DB; ++db)
 #pragma unroll
-            for (int bq = 0; bq < 4; ++bq)
-                st16(dst + (32 * db + 8 * bq + 4 * hw) * 4,
-                     gated(a, f32x4{acc[db][4 * bq], acc[db][4 * bq + 1], acc[db][4 * bq + 2], acc[db][4 * bq + 3]} * inv,
-                           gate_load(a, s, jw, hd, 32 * db + 8 * bq + 4 * hw)));
+            for (int bq = 0; bq < 4; ++bq) {
+                const int d = 32 * db + 8 * bq + 4 * hw;
+                f32x4 o = f32x4{acc[db][4 * bq], acc[db][4 * bq + 1], acc[db][4 * bq + 2], acc[db][4 * bq + 3]} * inv;
+                if (!share) o = gated(a, o, gate_load(a, s, jw, hd, d));
+                st16(dst + d * 4, o);
+            }
     }
 }
 
@@ -815,7 +824,7 @@ __global__ __launch_bounds__(kThreads, PfDim<D>::GROUPS) void prefill_gated(FaAr
     const bool lengths = mask_rows_block_causal(a, reinterpret_cast<int*>(&sh));
     if constexpr (GATE == 0) {
         if (lengths)
-            prefill_body<MODE_FAST, D, KV, QQ8>(mask_as_lengths(a), 1, nrb, n_cu, sh.fast);
+            prefill_body<MODE_FAST, D, KV, QQ8, true>(mask_as_lengths(a), 1, nrb, n_cu, sh.fast);
         else
             prefill_body<MODE_MASK, D, KV, QQ8>(a, 0, nrb, n_cu, sh.mask);
     } else {
