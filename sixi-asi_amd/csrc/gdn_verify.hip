@@ -46,6 +46,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "gdn_internal.hpp"
 
@@ -679,164 +680,169 @@ __global__ __launch_bounds__(512) void gdn_scan_kernel(GdnArgs a, int grouped) {
         return;
     }
 
-    // ---- producers ----
-    const int pw = wv - 4;
-    const int half = pw & 1;
-    const bool is_q = pw >= 2;
-    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    const char* const kb = a.k + (int64_t)g * a.k_nb1 + (int64_t)s * a.k_nb3 + 256 * half + 16 * gl;
-    const char* const qb = a.q + (int64_t)g * a.q_nb1 + (int64_t)s * a.q_nb3 + 256 * half + 16 * gl;
-    // a chunk in registers: row lr, columns 64 half + 16 m + 4 gl .. + 3 (zeros past the block); in
-    // wave 7 also the gates of row lr (1 and 0 past the block) and rows lane / 8, 8 + lane / 8 of v
-    struct Chunk {
-        f32x4 k[4], q[4], v[2];
-        float al, be;
-    };
-    auto load_rows = [&](int c, Chunk& x) {
-        const int t = c * T + lr;
+    // ---- producers ---- (one loop for each wave: a common one holds more than the SGPRs)
+    auto produce = [&](auto PW) {
+        constexpr int pw = decltype(PW)::value, half = pw & 1;
+        constexpr bool is_q = pw >= 2;
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        const char* const kb = a.k + (int64_t)g * a.k_nb1 + (int64_t)s * a.k_nb3 + 256 * half + 16 * gl;
+        const char* const qb = a.q + (int64_t)g * a.q_nb1 + (int64_t)s * a.q_nb3 + 256 * half + 16 * gl;
+        // a chunk in registers: row lr, columns 64 half + 16 m + 4 gl .. + 3 (zeros past the block); in
+        // wave 7 also the gates of row lr (1 and 0 past the block) and rows lane / 8, 8 + lane / 8 of v
+        struct Chunk {
+            f32x4 k[4], q[4], v[2];
+            float al, be;
+        };
+        auto load_rows = [&](int c, Chunk& x) {
+            const int t = c * T + lr;
 #pragma unroll
-        for (int m = 0; m < 4; ++m) x.k[m] = x.q[m] = zero;
-        if (t < ql) {
+            for (int m = 0; m < 4; ++m) x.k[m] = x.q[m] = zero;
+            if (t < ql) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                x.k[m] = *reinterpret_cast<const f32x4*>(kb + (int64_t)t * a.k_nb2 + 64 * m);
-                if (is_q) x.q[m] = *reinterpret_cast<const f32x4*>(qb + (int64_t)t * a.q_nb2 + 64 * m);
+                for (int m = 0; m < 4; ++m) {
+                    x.k[m] = *reinterpret_cast<const f32x4*>(kb + (int64_t)t * a.k_nb2 + 64 * m);
+                    if (is_q) x.q[m] = *reinterpret_cast<const f32x4*>(qb + (int64_t)t * a.q_nb2 + 64 * m);
+                }
             }
-        }
-    };
-    auto load_gates = [&](int c, Chunk& x) {
-        const int t = c * T + lr;
-        x.al = 1.0f;
-        x.be = 0.0f;
-        if (t < ql) {
-            x.al = *reinterpret_cast<const float*>(a.alpha + (int64_t)g * a.a_nb0 + (int64_t)t * a.a_nb1 + (int64_t)s * a.a_nb2);
-            x.be = *reinterpret_cast<const float*>(a.beta + (int64_t)g * a.b_nb0 + (int64_t)t * a.b_nb1 + (int64_t)s * a.b_nb2);
-        }
+        };
+        auto load_gates = [&](int c, Chunk& x) {
+            const int t = c * T + lr;
+            x.al = 1.0f;
+            x.be = 0.0f;
+            if (t < ql) {
+                x.al = *reinterpret_cast<const float*>(a.alpha + (int64_t)g * a.a_nb0 + (int64_t)t * a.a_nb1 + (int64_t)s * a.a_nb2);
+                x.be = *reinterpret_cast<const float*>(a.beta + (int64_t)g * a.b_nb0 + (int64_t)t * a.b_nb1 + (int64_t)s * a.b_nb2);
+            }
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int tv = c * T + 8 * u + (lane >> 3);
-            x.v[u] = zero;
-            if (tv < ql)
-                x.v[u] = *reinterpret_cast<const f32x4*>(a.v + (int64_t)g * a.v_nb1 + (int64_t)tv * a.v_nb2 +
-                                                         (int64_t)s * a.v_nb3 + 4 * hr0 + 16 * (lane & 7));
-        }
-    };
-    // M = (I + L)^-1 by blocks: the 4 x 4 diagonal blocks in closed form (D), then twice
-    // M <- M - M Lo M with Lo the blocks below the diagonal of the doubled blocks, on the matrix
-    // cores (elimination row by row in one wave took 0.6 us of a 2.8 us iteration).  A product's
-    // accumulator layout is its B operand's: lane = column lr, rows 4 gl + j.
-    auto invert = [&](float (&L)[T][T], float (&M)[T][T]) {
-        const int bk = lr >> 2, p = lr & 3;
-        const f32x4 l1 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 1][4 * bk]);
-        const f32x4 l2 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 2][4 * bk]);
-        const f32x4 l3 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 3][4 * bk]);
-        const f32x4 lx = *reinterpret_cast<const f32x4*>(&L[lr][4 * gl]);
-        const float m10 = -l1[0], m21 = -l2[1], m32 = -l3[2];
-        const float m20 = -fmaf(l2[1], m10, l2[0]), m31 = -fmaf(l3[2], m21, l3[1]);
-        const float m30 = -fmaf(l3[2], m20, fmaf(l3[1], m10, l3[0]));
-        const bool diag = gl == bk;
-        f32x4 row = p == 0 ? f32x4{1.0f, 0.0f, 0.0f, 0.0f} : p == 1 ? f32x4{m10, 1.0f, 0.0f, 0.0f}
-                  : p == 2 ? f32x4{m20, m21, 1.0f, 0.0f} : f32x4{m30, m31, m32, 1.0f};
-        f32x4 col = p == 0 ? f32x4{1.0f, m10, m20, m30} : p == 1 ? f32x4{0.0f, 1.0f, m21, m31}
-                  : p == 2 ? f32x4{0.0f, 0.0f, 1.0f, m32} : f32x4{0.0f, 0.0f, 0.0f, 1.0f};
-        row = diag ? row : zero;  // D[lr][4 gl + j]
-        col = diag ? col : zero;  // D[4 gl + j][lr]
-        const f32x4 lo4 = gl + 1 == bk && (bk & 1) ? lx : zero;
-        const f32x4 lo8 = gl < 2 && bk >= 2 ? lx : zero;
-        f32x4 x = zero, m8 = col;
+            for (int u = 0; u < 2; ++u) {
+                const int tv = c * T + 8 * u + (lane >> 3);
+                x.v[u] = zero;
+                if (tv < ql)
+                    x.v[u] = *reinterpret_cast<const f32x4*>(a.v + (int64_t)g * a.v_nb1 + (int64_t)tv * a.v_nb2 +
+                                                             (int64_t)s * a.v_nb3 + 4 * hr0 + 16 * (lane & 7));
+            }
+        };
+        // M = (I + L)^-1 by blocks: the 4 x 4 diagonal blocks in closed form (D), then twice
+        // M <- M - M Lo M with Lo the blocks below the diagonal of the doubled blocks, on the matrix
+        // cores (elimination row by row in one wave took 0.6 us of a 2.8 us iteration).  A product's
+        // accumulator layout is its B operand's: lane = column lr, rows 4 gl + j.
+        auto invert = [&](float (&L)[T][T], float (&M)[T][T]) {
+            const int bk = lr >> 2, p = lr & 3;
+            const f32x4 l1 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 1][4 * bk]);
+            const f32x4 l2 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 2][4 * bk]);
+            const f32x4 l3 = *reinterpret_cast<const f32x4*>(&L[4 * bk + 3][4 * bk]);
+            const f32x4 lx = *reinterpret_cast<const f32x4*>(&L[lr][4 * gl]);
+            const float m10 = -l1[0], m21 = -l2[1], m32 = -l3[2];
+            const float m20 = -fmaf(l2[1], m10, l2[0]), m31 = -fmaf(l3[2], m21, l3[1]);
+            const float m30 = -fmaf(l3[2], m20, fmaf(l3[1], m10, l3[0]));
+            const bool diag = gl == bk;
+            f32x4 row = p == 0 ? f32x4{1.0f, 0.0f, 0.0f, 0.0f} : p == 1 ? f32x4{m10, 1.0f, 0.0f, 0.0f}
+                      : p == 2 ? f32x4{m20, m21, 1.0f, 0.0f} : f32x4{m30, m31, m32, 1.0f};
+            f32x4 col = p == 0 ? f32x4{1.0f, m10, m20, m30} : p == 1 ? f32x4{0.0f, 1.0f, m21, m31}
+                      : p == 2 ? f32x4{0.0f, 0.0f, 1.0f, m32} : f32x4{0.0f, 0.0f, 0.0f, 1.0f};
+            row = diag ? row : zero;  // D[lr][4 gl + j]
+            col = diag ? col : zero;  // D[4 gl + j][lr]
+            const f32x4 lo4 = gl + 1 == bk && (bk & 1) ? lx : zero;
+            const f32x4 lo8 = gl < 2 && bk >= 2 ? lx : zero;
+            f32x4 x = zero, m8 = col;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x = mma4(lo4[j], col[j], x);
+            for (int j = 0; j < 4; ++j) x = mma4(lo4[j], col[j], x);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) m8 = mma4(-row[j], x[j], m8);
+            for (int j = 0; j < 4; ++j) m8 = mma4(-row[j], x[j], m8);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) M[4 * gl + j][lr] = m8[j];
-        x = zero;
+            for (int j = 0; j < 4; ++j) M[4 * gl + j][lr] = m8[j];
+            x = zero;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x = mma4(lo8[j], m8[j], x);
-        const f32x4 mrow = *reinterpret_cast<const f32x4*>(&M[lr][4 * gl]);
-        f32x4 m16 = m8;
+            for (int j = 0; j < 4; ++j) x = mma4(lo8[j], m8[j], x);
+            const f32x4 mrow = *reinterpret_cast<const f32x4*>(&M[lr][4 * gl]);
+            f32x4 m16 = m8;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) m16 = mma4(-mrow[j], x[j], m16);
+            for (int j = 0; j < 4; ++j) m16 = mma4(-mrow[j], x[j], m16);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) M[4 * gl + j][lr] = m16[j];
-    };
-    f32x4 gr = zero;  // this wave's Gram product of chunk i + 2, then of chunk i + 3
-    // iteration i; x holds chunk i + 3 and takes chunk i + 5
-    auto iteration = [&](int i, Chunk& x) {
-        if (half == 0 && i + 2 >= 0 && i + 2 < n_chunks) {
-            const int b4 = (i + 2) & 3, b2 = i & 1;
-            gr += sh.G[is_q][lane];  // k_{4gl+r} . k_lr (or . q_lr)
-            if (is_q) {
-                const f32x4 ex = *reinterpret_cast<const f32x4*>(&sh.E[b4][lr][4 * gl]);
-                *reinterpret_cast<f32x4*>(&sh.W[b4][lr][4 * gl]) = ex * gr;  // 0 past the diagonal
-            } else {
+            for (int j = 0; j < 4; ++j) M[4 * gl + j][lr] = m16[j];
+        };
+        f32x4 gr = zero;  // this wave's Gram product of chunk i + 2, then of chunk i + 3
+        // iteration i; x holds chunk i + 3 and takes chunk i + 5
+        auto iteration = [&](int i, Chunk& x) {
+            if (half == 0 && i + 2 >= 0 && i + 2 < n_chunks) {
+                const int b4 = (i + 2) & 3, b2 = i & 1;
+                gr += sh.G[is_q][lane];  // k_{4gl+r} . k_lr (or . q_lr)
+                if (is_q) {
+                    const f32x4 ex = *reinterpret_cast<const f32x4*>(&sh.E[b4][lr][4 * gl]);
+                    *reinterpret_cast<f32x4*>(&sh.W[b4][lr][4 * gl]) = ex * gr;  // 0 past the diagonal
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int t = 4 * gl + r;
+                        float l = 0.0f;
+                        if (lr < t) l = sh.B[b4][t] * (DECAY_FIRST ? sh.E[b4][t][lr] : sh.E[b4][t - 1][lr]) * gr[r];
+                        sh.L[b2][t][lr] = l;
+                    }
+                }
+            }
+            if (pw == 1 && i + 1 >= 0 && i + 1 < n_chunks) invert(sh.L[(i + 1) & 1], sh.M[(i + 1) & 1]);
+            const bool on = i + 3 < n_chunks;
+            if (pw == 3 && on) {
+                const int b4 = (i + 3) & 3;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) *reinterpret_cast<f32x4*>(&sh.v[b4][8 * u + (lane >> 3)][4 * (lane & 7)]) = x.v[u];
+                // column lr of E, multiplied in row order; this lane's rows 4 gl .. + 3
+                float e = 1.0f, ev[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                const int ai = __builtin_bit_cast(int, x.al);
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const float at = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, t));
+                    if (t > lr) e *= at;
+                    if (gl == t / 4) ev[t % 4] = t >= lr ? e : 0.0f;
+                }
+                const float a0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, 0));
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int t = 4 * gl + r;
-                    float l = 0.0f;
-                    if (lr < t) l = sh.B[b4][t] * (DECAY_FIRST ? sh.E[b4][t][lr] : sh.E[b4][t - 1][lr]) * gr[r];
-                    sh.L[b2][t][lr] = l;
+                    sh.E[b4][t][lr] = ev[r];
+                    if (lr == 0) {
+                        sh.A[b4][t] = ev[r] * a0;
+                        if (DECAY_FIRST) sh.C[b4][t] = ev[r] * a0;
+                        else if (t + 1 < T) sh.C[b4][t + 1] = ev[r] * a0;
+                    }
                 }
+                if (!DECAY_FIRST && lane == 0) sh.C[b4][0] = 1.0f;
+                if (gl == 0) sh.B[b4][lr] = x.be;
+                if (i + 5 < n_chunks) load_gates(i + 5, x);
             }
-        }
-        if (pw == 1 && i + 1 >= 0 && i + 1 < n_chunks) invert(sh.L[(i + 1) & 1], sh.M[(i + 1) & 1]);
-        const bool on = i + 3 < n_chunks;
-        if (pw == 3 && on) {
-            const int b4 = (i + 3) & 3;
+            lds_barrier();
+            if (on) {
+                const int b3 = (i + 3) % 3;
+                f32x4 g2[2] = {zero, zero};
 #pragma unroll
-            for (int u = 0; u < 2; ++u) *reinterpret_cast<f32x4*>(&sh.v[b4][8 * u + (lane >> 3)][4 * (lane & 7)]) = x.v[u];
-            // column lr of E, multiplied in row order; this lane's rows 4 gl .. + 3
-            float e = 1.0f, ev[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            const int ai = __builtin_bit_cast(int, x.al);
+                for (int m = 0; m < 4; ++m) {
+                    *reinterpret_cast<f32x4*>(is_q ? &sh.q[b3][lr][64 * half + 16 * m + 4 * gl]
+                                                   : &sh.k[b3][lr][64 * half + 16 * m + 4 * gl]) = is_q ? x.q[m] : x.k[m];
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const float at = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, t));
-                if (t > lr) e *= at;
-                if (gl == t / 4) ev[t % 4] = t >= lr ? e : 0.0f;
-            }
-            const float a0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(ai, 0));
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 4 * gl + r;
-                sh.E[b4][t][lr] = ev[r];
-                if (lr == 0) {
-                    sh.A[b4][t] = ev[r] * a0;
-                    if (DECAY_FIRST) sh.C[b4][t] = ev[r] * a0;
-                    else if (t + 1 < T) sh.C[b4][t + 1] = ev[r] * a0;
+                    for (int j = 0; j < 4; ++j) g2[m & 1] = mma4(x.k[m][j], is_q ? x.q[m][j] : x.k[m][j], g2[m & 1]);
                 }
+                gr = g2[0] + g2[1];
+                if (half) sh.G[is_q][lane] = gr;
+                if (i + 5 < n_chunks) load_rows(i + 5, x);
             }
-            if (!DECAY_FIRST && lane == 0) sh.C[b4][0] = 1.0f;
-            if (gl == 0) sh.B[b4][lr] = x.be;
-            if (i + 5 < n_chunks) load_gates(i + 5, x);
+            lds_barrier();
+        };
+        Chunk even, odd;
+        load_rows(0, even);
+        load_rows(1, odd);
+        if (pw == 3) {
+            load_gates(0, even);
+            load_gates(1, odd);
         }
-        lds_barrier();
-        if (on) {
-            const int b3 = (i + 3) % 3;
-            f32x4 g2[2] = {zero, zero};
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                *reinterpret_cast<f32x4*>(is_q ? &sh.q[b3][lr][64 * half + 16 * m + 4 * gl]
-                                               : &sh.k[b3][lr][64 * half + 16 * m + 4 * gl]) = is_q ? x.q[m] : x.k[m];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) g2[m & 1] = mma4(x.k[m][j], is_q ? x.q[m][j] : x.k[m][j], g2[m & 1]);
-            }
-            gr = g2[0] + g2[1];
-            if (half) sh.G[is_q][lane] = gr;
-            if (i + 5 < n_chunks) load_rows(i + 5, x);
+        for (int i = -3; i < n_chunks; i += 2) {
+            iteration(i, even);
+            if (i + 1 < n_chunks) iteration(i + 1, odd);
         }
-        lds_barrier();
     };
-    Chunk even, odd;
-    load_rows(0, even);
-    load_rows(1, odd);
-    if (pw == 3) {
-        load_gates(0, even);
-        load_gates(1, odd);
-    }
-    for (int i = -3; i < n_chunks; i += 2) {
-        iteration(i, even);
-        if (i + 1 < n_chunks) iteration(i + 1, odd);
-    }
+    if (wv == 4) produce(std::integral_constant<int, 0>{});
+    else if (wv == 5) produce(std::integral_constant<int, 1>{});
+    else if (wv == 6) produce(std::integral_constant<int, 2>{});
+    else produce(std::integral_constant<int, 3>{});
 }
 
 // Work-groups of the chunked kernel that fit the device at once (each then runs several items).
@@ -894,7 +900,7 @@ template <int HD>
 hipError_t launch_chunked(const GdnArgs& a, hipStream_t stream) {
     // While its work-groups fit the CUs at once the scan kernel is the faster one at every length (48
     // groups, one stream: 4 rows 9.4 -> 8.7 us, 16 rows 9.6 -> 9.0, 33 rows 18.1 -> 15.0, 2048 rows
-    // 741 -> 337 with the launch); beyond that its eight waves per CU lose to the sixteen of the chunked kernel (two
+    // 674 -> 325); beyond that its eight waves per CU lose to the sixteen of the chunked kernel (two
     // streams, an earlier form of it: 16 rows 10.1 against 15.0 us, 128 rows 46 against 55).
     if ((int64_t)a.S * a.G * (HD / kScanRows) <= cu_count()) return launch_scan<HD>(a, stream);
     return a.decay_first ? launch_chunked_df<HD, true>(a, stream) : launch_chunked_df<HD, false>(a, stream);
