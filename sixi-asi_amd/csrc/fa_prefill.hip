@@ -742,7 +742,7 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
 
 // Adds up the shares of split items: out = sum_c w_c O_c / sum_c w_c l_c with w_c = 2^(m_c - max m).
 // One thread per four dims of a row; a share that saw no cell of the row has m = -inf and zero sums.
-// Moves bytes only: C x 4 D read and 4 D written per row.
+// Moves bytes only: C x 4 D read and 4 D written per row (HBM- and launch-bound).
 template <int D>
 __global__ __launch_bounds__(kThreads) void prefill_merge(FaArgs a) {
     constexpr int TPR = D / 4, RPB = kThreads / TPR;  // threads per row, rows per work-group
@@ -899,7 +899,14 @@ hipError_t launch_prefill_d(const FaArgs& a, int mask_mode, hipStream_t stream) 
 // through memory costs.  A share walks n / C tiles and costs kStart tiles of start-up (Q, the
 // first tile, the sums' way out); its sums cross memory twice (kMerge tiles' time over the whole
 // chip).  Every C up to 16 whose launch stays within two full rounds is priced by its rounds; n_kv
-// stands in for the lengths, which only the device knows.
+// stands in for the lengths, which only the device knows.  Measured at one share and more (us, the
+// last one is what the rule takes):
+//   1 x 173 rows behind 11400 cells, 256 dims f16   1: 552   4: 157   6: 114   7: 101
+//   4 x 40 rows behind 12000 cells, 256 dims        1: 577   4: 164   6: 118   8: 97
+//   1 x 300 rows behind 20000 cells, 128 dims       1: 413   4: 118   6: 108   8: 97
+//   1 x 64 rows behind 4000 cells, 128 dims         1: 87    4: 32    8: 24.8  10: 25.4
+//   1 x 600 rows behind 2000 cells, 256 dims        1: 132   2: 88
+//   1 x 17 rows behind 300 cells, 128 dims          1: 12.9  2: 13.2
 int prefill_split(int64_t blocks, int64_t n_kv, int head_dim, int cu_count) {
     if (2 * blocks > cu_count) return 1;
     constexpr double kStart = 4.0;
