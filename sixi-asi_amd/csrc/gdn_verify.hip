@@ -529,9 +529,10 @@ __global__ __launch_bounds__(256) void gdn_verify_chunked_kernel(GdnArgs a, int 
 //     wave 7 stages v, the gates and their products E of chunk i + 3, wave 5 inverts I + L of chunk
 //     i + 1.  Each issues the global loads of its chunk two iterations ahead.
 // Every SIMD holds one consumer and one producer, whose 56 and 16 f32 MFMAs (32 cycles each) per
-// iteration are its floor: 2304 cycles, 123 us over the 128 chunks of 2048 rows, which take 325 us:
-// the producers switched off leave 219 (the consumers' chain P -> exchange -> U -> state), the
-// inversion alone is 35 of it, the staging loads 28, E 27, k k^T and k q^T 24.
+// iteration are its floor: 2304 cycles, 123 us over the 128 chunks of 2048 rows, which take 307 us
+// (a call; 739 with the chunked kernel).  Before each producer wave had a loop of its own it took 325
+// in graph replays, of which the producers switched off left 219 (the consumers' chain P -> exchange
+// -> U -> state); the inversion was 35 of it, the staging loads 28, E 27, k k^T and k q^T 24.
 constexpr int kScanRows = 32;
 
 struct GdnScanLds {
