@@ -722,7 +722,9 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
         if (share) {
             float* slot = a.part + (int64_t)(chunk + a.pf_split * (g + a.Hkv * (s + a.S * rb))) * PrefillSlot<D>::FLOATS;
             if (hw == 0) {
-                slot[PrefillSlot<D>::M + rw] = RAW ? m_ref * c2 : m_ref;
+                // (no reference yet: -inf if the share saw no cell of the row, else -- c2 = 0, whose
+                // threshold nothing exceeds -- the 0 that its probabilities were taken against)
+                slot[PrefillSlot<D>::M + rw] = m_ref == neg_inf() ? (l_sum == 0.0f ? neg_inf() : 0.0f) : RAW ? m_ref * c2 : m_ref;
                 slot[PrefillSlot<D>::L + rw] = l_sum;
             }
             inv = 1.0f;

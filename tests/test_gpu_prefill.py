@@ -208,3 +208,24 @@ def test_split_row_blocks(fa, kv_len, q_len, H, Hkv, D, kv, mode):
     if mode in ("lengths", "causal"):
         want = oracle.attention_for_workload(host, w.kv_type)
         _check(np.concatenate([want[s, :q_len[s]].ravel() for s in range(w.S)]), got, "split")
+
+
+@pytest.mark.parametrize("D", [128, 256])
+def test_split_row_blocks_at_scale_0(fa, D):
+    """A scale of 0 weighs every cell alike: each output is the mean of V, split as unsplit.  One
+    stream fills the cache, the other one tile of it, which most of its work-groups see nothing of;
+    no mask, so every tile is whole.  Against 64 bits."""
+    _say(f"split scale=0 D={D}")
+    S, n_q, H, Hkv, n_kv = 2, 22, 24, 4, 4096
+    cells = [n_kv, 64]
+    gen = torch.Generator(device="cuda").manual_seed(77)
+    q = 0.5 * torch.randn((S, n_q, H, D), generator=gen, device="cuda")
+    k, v = (torch.randn((S, n_kv, Hkv, D), generator=gen, device="cuda", dtype=torch.float16) for _ in range(2))
+    kv_len = torch.tensor([c - n_q for c in cells], dtype=torch.int32, device="cuda")
+    out = torch.full((S, n_q, H, D), float("nan"), dtype=torch.float32, device="cuda")
+    fa(q, k, v, out, kv_len=kv_len, mask_mode=sa.MASK_NONE, scale=0.0)
+    torch.cuda.synchronize()
+    got, v = out.cpu().numpy(), v.cpu().double().numpy()
+    for s in range(S):
+        mean = np.repeat(v[s, :cells[s]].mean(0), H // Hkv, axis=0)
+        _check(np.broadcast_to(mean, got[s].shape), got[s], f"stream {s}")
