@@ -73,7 +73,8 @@ enum {
 };
 
 /* sixi_attn_params.flags.  BOUNDED_WORKSPACE: never stage a q8_0 cache as f16 in the
- * workspace, so the workspace does not grow with the cache.  Without it, prefill-sized
+ * workspace, so the workspace does not grow with the cache (SPLIT_PREFILL's sums, if asked
+ * for, are bounded).  Without it, prefill-sized
  * blocks over a q8_0 cache stage K and V as f16 operands (the prefill kernel converts Q to
  * the q8_0 dot type itself; split-K calls of unaligned 256-dim rows also stage Q) while that
  * copy takes at most
@@ -91,6 +92,13 @@ enum {
  * sixi_attn_gate bit for bit, without that second pass over the output.  No counterpart in
  * ggml_flash_attn_ext (upstream runs the gate as a separate graph node). */
 #define SIXI_ATTN_FLAG_GATE 2
+/* SPLIT_PREFILL: the workspace is this call's alone while it runs, so a prefill-sized block whose
+ * row blocks leave CUs idle, over a long cache, may share the cells of each row block among several
+ * work-groups, which leave f32 sums there (at most 16 per row block and two launch rounds, whatever
+ * the cache length).  sixi_attn_workspace_bytes then includes the sums.  Without it such a call runs
+ * one work-group per row block and writes no workspace beyond a q8_0 cache's staging and an explicit
+ * mask's table.  Other calls do not depend on it. */
+#define SIXI_ATTN_FLAG_SPLIT_PREFILL 8
 
 /* ggml-compatible strided view.  ne[0] is the innermost extent (elements); nb[] are byte
  * strides; for q8_0, nb[0] = 34 (one 32-element block) and a row of ne[0] elements takes
@@ -121,8 +129,7 @@ typedef struct sixi_attn_params {
     float max_bias;         /* ALiBi; 0 = off                                              */
     float logit_softcap;    /* 0 = off                                                     */
     float reserved_f;
-    void* workspace;        /* device scratch of >= sixi_attn_workspace_bytes() bytes
-                               (or the least of sixi_attn_workspace_range()),
+    void* workspace;        /* device scratch of >= sixi_attn_workspace_bytes() bytes,
                                256-byte aligned; its contents need no initialisation       */
     size_t workspace_bytes;
     void* stream;           /* hipStream_t; NULL = the null stream                         */
@@ -151,7 +158,9 @@ int sixi_attn_forward(const sixi_attn_params* p);
  * until the process ends; `workspace` and `workspace_bytes` are ignored.  q8_0 caches are
  * staged only while the staging fits the scratch (as with SIXI_ATTN_FLAG_BOUNDED_WORKSPACE
  * beyond that).  A description whose scratch (split-K partials, a q8_0 staging that cannot
- * be avoided) exceeds that size returns SIXI_E_OUT_OF_BOUNDS before any launch.  The scratch needs no initialisation, but every
+ * be avoided) exceeds that size returns SIXI_E_OUT_OF_BOUNDS before any launch.  With
+ * SIXI_ATTN_FLAG_SPLIT_PREFILL as many work-groups share a row block as leave their sums in
+ * the scratch.  The scratch needs no initialisation, but every
  * call on a GPU shares it: calls that may overlap on one GPU (different streams, or
  * threads without ordering) race; order them on one stream. */
 #define SIXI_ATTN_NOALLOC_SCRATCH_BYTES ((size_t)32 << 20)
@@ -161,12 +170,8 @@ int sixi_attn_forward_noalloc(const sixi_attn_params* p);
  * the device's CU count; not on the device-side lengths). */
 int sixi_attn_workspace_bytes(const sixi_attn_params* p, size_t* bytes);
 
-/* The least workspace the call runs with, beside the size above.  The two differ for prefill-sized
- * blocks too few to fill the GPU, over a long cache: with the full size several work-groups share
- * the cells of each row block and leave f32 sums in the workspace (at most 16 per row block and two
- * launch rounds, whatever the cache length), with less fewer do, down to none.  The workspace is the
- * call's own while it runs, so calls that may overlap need one each; a call given only `least` bytes
- * of an f16 cache's prefill writes none of it. */
+/* The size above without SIXI_ATTN_FLAG_SPLIT_PREFILL (`least`) and with it (`bytes`), whether or
+ * not `p` has the flag: equal unless the flag splits the call's row blocks. */
 int sixi_attn_workspace_range(const sixi_attn_params* p, size_t* least, size_t* bytes);
 
 /* Host-side validation only (no device access): SIXI_OK or the error forward() returns. */

@@ -77,7 +77,7 @@ struct Plan {
     bool mask_prepass = false; // explicit mask reduced to per-row offsets first (fa_mask.hip)
     size_t prepass_offset = 0; // byte offset of its table (S * n_q int32), after the rest
     size_t ws_bytes = 0;
-    size_t ws_min = 0;         // the least a call can run with (ws_bytes without the prefill split)
+    size_t ws_min = 0;         // ws_bytes without the prefill split
     size_t part_offset = 0;    // prefill split: byte offset of its sums (after the staging area)
 };
 
@@ -103,7 +103,7 @@ void prepass_layout(Plan& pl) {
     pl.ws_bytes = pl.prepass_offset + align_up((size_t)pl.a.S * pl.a.n_q * sizeof(int32_t), kWsAlign);
 }
 
-// Fewer shares per row block until the workspace fits in `bytes` (down to none).
+// Fewer shares per row block until the workspace fits in `bytes` (down to one: no split).
 void prefill_fit(Plan& pl, size_t bytes) {
     while (!pl.splitk && pl.a.pf_split > 1 && pl.ws_bytes > bytes) prefill_layout(pl, pl.a.pf_split - 1);
 }
@@ -134,7 +134,8 @@ void splitk_layout(Plan& pl, int64_t slots) {
 // avoided: 256-dim rows that are not 16-byte aligned).
 int resolve(const sixi_attn_params* p, Plan* out, size_t stage_cap = SIXI_ATTN_STAGE_CAP_BYTES) {
     if (!p || !out) return SIXI_E_INVALID_ARGUMENT;
-    if ((p->flags & ~(SIXI_ATTN_FLAG_BOUNDED_WORKSPACE | SIXI_ATTN_FLAG_GATE)) != 0) return SIXI_E_INVALID_ARGUMENT;
+    constexpr int32_t kFlags = SIXI_ATTN_FLAG_BOUNDED_WORKSPACE | SIXI_ATTN_FLAG_GATE | SIXI_ATTN_FLAG_SPLIT_PREFILL;
+    if ((p->flags & ~kFlags) != 0) return SIXI_E_INVALID_ARGUMENT;
     if (p->flags & SIXI_ATTN_FLAG_BOUNDED_WORKSPACE) stage_cap = 0;
     const sixi_view &q = p->q, &k = p->k, &v = p->v, &o = p->out;
     if (!q.data || !k.data || !v.data || !o.data) return SIXI_E_INVALID_ARGUMENT;
@@ -377,7 +378,8 @@ int resolve(const sixi_attn_params* p, Plan* out, size_t stage_cap = SIXI_ATTN_S
     } else {
         if (S * H * ((n_q + 127) / 128) > (int64_t)INT32_MAX) return SIXI_E_UNSUPPORTED;
         const int64_t blocks = S * Hkv * sixi::prefill_row_blocks(n_q, a.G);
-        prefill_layout(pl, sixi::prefill_split(blocks, n_kv, pl.D, cu_count_cached()));
+        const bool may_split = (p->flags & SIXI_ATTN_FLAG_SPLIT_PREFILL) != 0;
+        prefill_layout(pl, may_split ? sixi::prefill_split(blocks, n_kv, pl.D, cu_count_cached()) : 1);
     }
     if (pl.splitk) {
         prepass_layout(pl);
@@ -488,9 +490,11 @@ int sixi_attn_workspace_bytes(const sixi_attn_params* p, size_t* bytes) {
 }
 
 int sixi_attn_workspace_range(const sixi_attn_params* p, size_t* least, size_t* bytes) {
-    if (!least || !bytes) return SIXI_E_INVALID_ARGUMENT;
+    if (!p || !least || !bytes) return SIXI_E_INVALID_ARGUMENT;
+    sixi_attn_params split = *p;
+    split.flags |= SIXI_ATTN_FLAG_SPLIT_PREFILL;
     Plan pl;
-    const int rc = resolve(p, &pl);
+    const int rc = resolve(&split, &pl);
     if (rc != SIXI_OK) return rc;
     *least = pl.ws_min;
     *bytes = pl.ws_bytes;
@@ -501,8 +505,7 @@ int sixi_attn_forward(const sixi_attn_params* p) {
     Plan pl;
     int rc = resolve(p, &pl);
     if (rc != SIXI_OK) return rc;
-    if (!p->workspace || p->workspace_bytes < pl.ws_min) return SIXI_E_OUT_OF_BOUNDS;
-    prefill_fit(pl, p->workspace_bytes);
+    if (!p->workspace || p->workspace_bytes < pl.ws_bytes) return SIXI_E_OUT_OF_BOUNDS;
     if (!aligned(p->workspace, kWsAlign)) return SIXI_E_ALIGNMENT;
     // the kernels write the workspace while they read the views
     if (workspace_overlaps(p, p->workspace, pl.ws_bytes)) return SIXI_E_INVALID_ARGUMENT;

@@ -30,6 +30,7 @@ MASK_NONE, MASK_BLOCK_CAUSAL, MASK_EXPLICIT = 0, 1, 2
 # sixi_attn_params.flags; the f16 staging of a q8_0 cache stays under STAGE_CAP_BYTES
 FLAG_BOUNDED_WORKSPACE = 1
 FLAG_GATE = 2
+FLAG_SPLIT_PREFILL = 8
 STAGE_CAP_BYTES = 64 << 20
 # status codes (negated sixi_asi::ErrorCode, include/sixi_asi/common.hpp:40-67)
 OK = 0
@@ -414,17 +415,15 @@ class FlashAttnExt:
         least, n = ctypes.c_size_t(0), ctypes.c_size_t(0)
         rc = self.lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(n))
         if rc == OK:
-            size = None
             if workspace is not None:
                 ws = workspace
-            elif least.value == n.value:
-                ws = self._workspace(n.value)
-            elif stream is None and not torch.cuda.is_current_stream_capturing():
+            elif least.value < n.value and stream is None and not torch.cuda.is_current_stream_capturing():
                 ws = self._split_workspace(p.stream, n.value)
+                p.flags |= FLAG_SPLIT_PREFILL
             else:
-                ws, size = self._workspace(least.value), least.value
+                ws = self._workspace(least.value)
             p.workspace = ws.data_ptr()
-            p.workspace_bytes = ws.numel() * ws.element_size() if size is None else size
+            p.workspace_bytes = ws.numel() * ws.element_size()
             rc = self.lib.sixi_attn_forward(ctypes.byref(p))
         if check and rc != OK:
             raise SixiAttnError(rc, strerror(rc))

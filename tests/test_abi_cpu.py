@@ -215,6 +215,33 @@ def test_workspace_must_not_overlap_the_views():
         assert lib.sixi_attn_forward(ctypes.byref(p)) == sa.E_INVALID_ARGUMENT, where
 
 
+def test_prefill_sums_only_on_request():
+    """A prefill whose row blocks could share their cells among idle CUs writes sums only with
+    FLAG_SPLIT_PREFILL: without it the workspace stays the token it is for one work-group per row
+    block, so one buffer may serve a prefill and other calls that overlap it."""
+    lib = sa.load_library()
+    for kw in ({}, {"D": 256}, {"kv_type": sa.TYPE_Q8_0}):
+        p = _params(S=1, n_q=64, n_kv=8192, **kw)
+        n, least, full = ctypes.c_size_t(0), ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert lib.sixi_attn_workspace_bytes(ctypes.byref(p), ctypes.byref(n)) == sa.OK
+        staging = 2 * 4 * 8192 * 256 if kw.get("kv_type") == sa.TYPE_Q8_0 else 0
+        assert n.value <= 4096 + staging
+        for flags in (0, sa.FLAG_SPLIT_PREFILL):
+            p.flags = flags
+            assert lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(full)) == sa.OK
+            assert least.value == n.value < full.value
+        assert lib.sixi_attn_workspace_bytes(ctypes.byref(p), ctypes.byref(n)) == sa.OK
+        assert n.value == full.value
+        # with the flag the call needs all of it (refused before any launch)
+        p.workspace, p.workspace_bytes = ADDR["ws"], full.value - 1
+        assert lib.sixi_attn_forward(ctypes.byref(p)) == sa.E_OUT_OF_BOUNDS
+    # blocks that fill the GPU, and split-K calls, do not depend on the flag
+    for kw in ({"n_q": 2048, "S": 4}, {"n_q": 16}):
+        p = _params(**kw)
+        assert lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(full)) == sa.OK
+        assert least.value == full.value
+
+
 def _paged_params(S, stride, n_q=1, n_pages=1024):
     """A paged call: K and V pools of 256-cell pages, a page table of `stride` pages per stream."""
     p = _params(S=S, n_q=n_q)

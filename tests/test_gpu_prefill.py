@@ -6,6 +6,7 @@ f32-accumulator restatement of ggml's CPU flash_attn_ext.  At full chunk size th
 checks row slices: rows [a, b) of a chunk over kv_len cached cells are exactly a block of
 b - a rows over kv_len + a cached cells (same cells, same causal rule).
 """
+import ctypes
 import sys
 
 import numpy as np
@@ -157,6 +158,46 @@ def test_prefill_f16_queries(fa):
         _check(want[s, :w.q_len[s]], got[s, :w.q_len[s]], f"f16 Q stream {s}")
 
 
+def _forward(fa, p, split, ws=None):
+    """sixi_attn_forward of `p` with or without the split, on a workspace of its own full of NaN bits."""
+    least, full = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    assert fa.lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(full)) == sa.OK
+    assert least.value < full.value, "the case is meant to split"
+    if split:
+        p.flags |= sa.FLAG_SPLIT_PREFILL
+    if ws is None:
+        ws = torch.full((full.value if split else least.value,), 0xFF, dtype=torch.uint8, device="cuda")
+    p.stream = torch.cuda.current_stream().cuda_stream
+    p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+    rc = fa.lib.sixi_attn_forward(ctypes.byref(p))
+    assert rc == sa.OK, sa.strerror(rc)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("D", [128, 256])
+def test_prefill_writes_no_workspace_unless_asked(fa, D):
+    """Without FLAG_SPLIT_PREFILL an f16 prefill leaves the workspace as it is however large it is
+    (another call may be using it), and so also runs with one whose unused tail meets a view."""
+    _say(f"large workspace, no split D={D}")
+    w = wl.Workload("whole prefill", 0x51A7_5300 + D, 1, [3000], [40], D=D)
+    host = wl.make_host(w)
+    dev = wl.to_device(host)
+    out = torch.empty((1, 40, w.H, D), dtype=torch.float32, device="cuda")
+    p = fa.params(dev["q"], dev["k"], dev["v"], out, kv_len=dev["kv_len"], q_len=dev["q_len"])
+    ws = torch.full((64 << 20,), 0xA5, dtype=torch.uint8, device="cuda")
+    _forward(fa, p, False, ws)
+    assert bool(torch.all(ws == 0xA5))
+    want = oracle.attention_for_workload(host, w.kv_type)
+    _check(want, out.cpu().numpy(), "whole")
+    # the same queries behind 1 MB of workspace that is declared to run through them
+    tail = torch.zeros((1 << 20) + dev["q"].numel() * 4, dtype=torch.uint8, device="cuda")
+    q = tail[1 << 20:].view(torch.float32).view(dev["q"].shape)
+    q.copy_(dev["q"])
+    out2 = torch.empty_like(out)
+    _forward(fa, fa.params(q, dev["k"], dev["v"], out2, kv_len=dev["kv_len"], q_len=dev["q_len"]), False, tail)
+    assert torch.equal(out, out2)
+
+
 @pytest.mark.parametrize("kv_len,q_len,H,Hkv,D,kv,mode", [
     ([1500], [17], 24, 4, 128, sa.TYPE_F16, "lengths"),         # 102 rows: one row block, 6 of them empty
     ([700, 0, 5], [22, 17, 0], 24, 4, 256, sa.TYPE_F16, "lengths"),  # a second block of 4 rows; shares with no cell
@@ -168,11 +209,9 @@ def test_prefill_f16_queries(fa):
 ])
 def test_split_row_blocks(fa, kv_len, q_len, H, Hkv, D, kv, mode):
     """Few row blocks over a long cache: several work-groups share the cells of each.  Against the
-    oracle (the bar above), and against the same call with the least workspace (no split): the two
+    oracle (the bar above), and against the same call without the flag (no split): the two
     differ by the order of f32 sums and the exponent references the f16 probabilities were taken
     against, 2^-11 of rounding each, averaged over the cells: a tenth of the bar's rel-L2 more."""
-    import ctypes
-
     _say(f"split kv_len={kv_len} q_len={q_len} H={H} Hkv={Hkv} D={D} kv={kv} {mode}")
     w = wl.Workload("split_prefill", 0x51A7_5100 + sum(q_len) + D, len(kv_len), kv_len, q_len, H=H, Hkv=Hkv, D=D, kv_type=kv)
     host = wl.make_host(w, poison=True)
@@ -192,12 +231,7 @@ def test_split_row_blocks(fa, kv_len, q_len, H, Hkv, D, kv, mode):
     for split in (True, False):
         out = torch.full((w.S, w.n_q, w.H, w.D), float("nan"), dtype=torch.float32, device="cuda")
         p = fa.params(dev["q"], dev["k"], dev["v"], out, **kw)
-        least, full = ctypes.c_size_t(0), ctypes.c_size_t(0)
-        assert fa.lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(full)) == sa.OK
-        assert least.value < full.value, "the case is meant to split"
-        ws = torch.full((full.value if split else least.value,), 0xFF, dtype=torch.uint8, device="cuda")
-        fa(dev["q"], dev["k"], dev["v"], out, workspace=ws, **kw)
-        torch.cuda.synchronize()
+        _forward(fa, p, split)
         outs.append(out.cpu().numpy())
     got, whole = (np.concatenate([o[s, :q_len[s]].ravel() for s in range(w.S)]) for o in outs)
     for s in range(w.S):  # rows past q_len are not written
@@ -229,3 +263,32 @@ def test_split_row_blocks_at_scale_0(fa, D):
     for s in range(S):
         mean = np.repeat(v[s, :cells[s]].mean(0), H // Hkv, axis=0)
         _check(np.broadcast_to(mean, got[s].shape), got[s], f"stream {s}")
+
+
+def test_split_in_the_fixed_scratch(fa):
+    """sixi_attn_forward_noalloc splits on request with as many shares as its 32 MiB hold: all of a small
+    call's, which then equals sixi_attn_forward bit for bit, and seven of the eight that 32 row blocks
+    at 256 dims would leave (33.8 MB); without the request it equals the unsplit call."""
+    for kv_len, q_len, D, fits in (([3000], [40], 128, True), ([12000, 500, 900, 40], [40, 40, 33, 40], 256, False)):
+        _say(f"noalloc split kv_len={kv_len} D={D}")
+        w = wl.Workload("noalloc split", 0x51A7_5400 + D, len(kv_len), kv_len, q_len, D=D)
+        host = wl.make_host(w, poison=True)
+        dev = wl.to_device(host)
+        want = oracle.attention_for_workload(host, w.kv_type)
+        for split in (True, False):
+            outs = []
+            for noalloc in (True, False):
+                out = torch.full((w.S, w.n_q, w.H, D), float("nan"), dtype=torch.float32, device="cuda")
+                p = fa.params(dev["q"], dev["k"], dev["v"], out, kv_len=dev["kv_len"], q_len=dev["q_len"])
+                if noalloc:
+                    p.flags |= sa.FLAG_SPLIT_PREFILL if split else 0
+                    p.stream = torch.cuda.current_stream().cuda_stream
+                    assert fa.lib.sixi_attn_forward_noalloc(ctypes.byref(p)) == sa.OK
+                    torch.cuda.synchronize()
+                else:
+                    _forward(fa, p, split)
+                outs.append(out.cpu().numpy())
+            same = np.array_equal(outs[0], outs[1], equal_nan=True)
+            assert same == (fits or not split)
+            for s in range(w.S):
+                _check(want[s, :q_len[s]], outs[0][s, :q_len[s]], f"stream {s} split={split}")
