@@ -316,8 +316,8 @@ class FlashAttnExt:
     """``ggml_flash_attn_ext`` over per-stream KV caches on one gfx950 GPU.
 
     Keeps a device workspace (grown on demand) so repeated calls allocate nothing; prefill calls that
-    split their row blocks over idle CUs keep one per stream beside it, so that a prefill may overlap
-    calls on other streams (under capture, or with an explicit ``stream``, they run unsplit).  A buffer
+    split their row blocks over idle CUs take one of their own from torch's allocator, so that they may
+    overlap other calls (under capture, or with an explicit ``stream``, they run unsplit).  A buffer
     that a larger call supersedes stays allocated for the life of the object, so a HIP graph
     captured over an earlier call still owns the memory its kernels write.  A caller may
     also pass its own ``workspace`` (a uint8 device tensor of at least
@@ -330,7 +330,6 @@ class FlashAttnExt:
         self.lib = load_library()
         self.device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
         self._ws = None
-        self._split_ws = {}  # stream -> workspace of the prefill calls that split their row blocks
         self._retired = []  # superseded workspaces: graphs captured before a regrowth still use them
 
     def params(self, q, k, v, out, kv_len=None, q_len=None, mask_mode=MASK_BLOCK_CAUSAL, mask=None,
@@ -385,15 +384,6 @@ class FlashAttnExt:
             self._ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=self.device)
         return self._ws
 
-    def _split_workspace(self, stream: int, nbytes: int):
-        import torch
-
-        ws = self._split_ws.get(stream)
-        if ws is None or ws.numel() < nbytes:
-            # (a superseded buffer goes back to the allocator, whose next use of it this stream orders)
-            ws = self._split_ws[stream] = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-        return ws
-
     def __call__(self, q, k, v, out, kv_len=None, q_len=None, mask_mode=MASK_BLOCK_CAUSAL, mask=None,
                  scale=None, max_bias=0.0, logit_softcap=0.0, kv_type=None, stream=None, check=True,
                  workspace=None, noalloc=False, page_table=None, bounded_workspace=False, gate=None) -> int:
@@ -418,7 +408,9 @@ class FlashAttnExt:
             if workspace is not None:
                 ws = workspace
             elif least.value < n.value and stream is None and not torch.cuda.is_current_stream_capturing():
-                ws = self._split_workspace(p.stream, n.value)
+                # the call's own until its kernels are queued (threads that share the stream may queue
+                # theirs in between), then the allocator's, which reuses it in this stream's order
+                ws = torch.empty(n.value, dtype=torch.uint8, device=self.device)
                 p.flags |= FLAG_SPLIT_PREFILL
             else:
                 ws = self._workspace(least.value)

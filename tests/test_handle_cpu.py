@@ -1,0 +1,94 @@
+"""FlashAttnExt's choice of workspaces on the host: the library sizes and validates the calls, a stand-in
+takes the launch, so that nothing here touches a device."""
+import ctypes
+import threading
+
+import pytest
+import torch
+
+import sixi_attn as sa
+
+STREAM = 0x5000
+
+
+class _Library:
+    """The library with sixi_attn_forward replaced by `launch(params)`."""
+
+    def __init__(self, launch):
+        self._lib, self._launch = sa.load_library(), launch
+        self.calls = []
+
+    def __getattr__(self, name):
+        fn = getattr(self._lib, name)
+        if name == "sixi_attn_forward":
+            def fn(ref):
+                self._launch(ref._obj)
+                return sa.OK
+
+        def call(*args):
+            self.calls.append(name)
+            return fn(*args)
+
+        return call
+
+
+@pytest.fixture
+def handle(monkeypatch):
+    state = {"capturing": False, "launch": lambda p: None}
+
+    class Stream:
+        cuda_stream = STREAM
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    fa = sa.FlashAttnExt(device="cpu")
+    fa.lib = _Library(lambda p: state["launch"](p))
+    return fa, state
+
+
+def _call(fa, rows=40, n_kv=4096, D=128, q8=False, **kw):
+    q = torch.zeros((1, rows, 24, D))
+    k = torch.zeros((1, n_kv, 4, D // 32 * 34), dtype=torch.uint8) if q8 else torch.zeros((1, n_kv, 4, D), dtype=torch.float16)
+    return fa(q, k, torch.zeros_like(k), torch.zeros((1, rows, 24, D)), kv_len=torch.zeros(1, dtype=torch.int32), **kw)
+
+
+def _held(fa):
+    """Bytes of the tensors the handle keeps."""
+    def walk(x):
+        if isinstance(x, torch.Tensor):
+            return x.numel() * x.element_size()
+        if isinstance(x, dict):
+            x = list(x.values())
+        return sum(map(walk, x)) if isinstance(x, (list, tuple)) else 0
+
+    return walk(vars(fa))
+
+
+def test_split_calls_of_two_threads_have_a_workspace_each(handle):
+    """Two threads on one stream may queue the kernels of two prefill calls in any order: the first one's
+    sums must not lie where the second one's will."""
+    fa, state = handle
+    _call(fa)
+    both = threading.Barrier(2, timeout=60)
+    ranges = []
+
+    def launch(p):
+        assert p.flags & sa.FLAG_SPLIT_PREFILL
+        ranges.append((p.workspace, p.workspace + p.workspace_bytes))
+        both.wait()  # both calls hold their workspace here
+
+    state["launch"] = launch
+    threads = [threading.Thread(target=_call, args=(fa,)) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    (a0, a1), (b0, b1) = ranges
+    assert a1 <= b0 or b1 <= a0
+
+
+def test_split_workspaces_are_given_back(handle):
+    fa, _ = handle
+    for stream_rows in (17, 40, 64, 100):
+        _call(fa, rows=stream_rows)
+    assert _held(fa) <= 4096
