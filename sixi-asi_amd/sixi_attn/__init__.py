@@ -411,6 +411,7 @@ class FlashAttnExt:
                 # the call's own until its kernels are queued (threads that share the stream may queue
                 # theirs in between), then the allocator's, which reuses it in this stream's order
                 ws = torch.empty(n.value, dtype=torch.uint8, device=self.device)
+                self._workspace(least.value)  # (sized here for the same call under capture)
                 p.flags |= FLAG_SPLIT_PREFILL
             else:
                 ws = self._workspace(least.value)

@@ -92,3 +92,18 @@ def test_split_workspaces_are_given_back(handle):
     for stream_rows in (17, 40, 64, 100):
         _call(fa, rows=stream_rows)
     assert _held(fa) <= 4096
+
+
+@pytest.mark.parametrize("q8", [False, True])
+def test_an_eager_split_call_sizes_what_the_captured_one_uses(handle, q8, monkeypatch):
+    """A captured call must allocate nothing: the eager call before it (which splits, and so runs on
+    another buffer) has sized the handle's workspace for it, a q8_0 cache's staging included."""
+    fa, state = handle
+    _call(fa, q8=q8)
+    kept = fa._ws
+    used = []
+    state.update(capturing=True, launch=lambda p: used.append((p.workspace, p.workspace_bytes, p.flags)))
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: pytest.fail("allocation under capture"))
+    _call(fa, q8=q8)
+    assert fa._ws is kept
+    assert used == [(kept.data_ptr(), kept.numel(), 0)]
