@@ -317,8 +317,7 @@ class FlashAttnExt:
 
     Keeps a device workspace (grown on demand) so repeated calls allocate nothing; prefill calls that
     split their row blocks over idle CUs take one of their own from torch's allocator, so that they may
-    overlap other calls (under capture, or with an explicit ``stream``, they run unsplit).  A buffer
-    that a larger call supersedes stays allocated for the life of the object, so a HIP graph
+    overlap other calls (``split_prefill`` of :meth:`__call__`).  A buffer that a larger call supersedes stays allocated for the life of the object, so a HIP graph
     captured over an earlier call still owns the memory its kernels write.  A caller may
     also pass its own ``workspace`` (a uint8 device tensor of at least
     :meth:`workspace_bytes`), e.g. one sized once before capture.
@@ -334,12 +333,14 @@ class FlashAttnExt:
 
     def params(self, q, k, v, out, kv_len=None, q_len=None, mask_mode=MASK_BLOCK_CAUSAL, mask=None,
                scale=None, max_bias=0.0, logit_softcap=0.0, kv_type=None, stream=None,
-               page_table=None, bounded_workspace=False, gate=None) -> SixiAttnParams:
+               page_table=None, bounded_workspace=False, gate=None, split_prefill=False) -> SixiAttnParams:
         """``page_table`` (an int32 device tensor [S, pages per stream]): k and v are page pools
         ``[n_pages, 256, Hkv, D]`` (uint8 q8_0 blocks as for a cache) read through it.
         ``bounded_workspace`` sets SIXI_ATTN_FLAG_BOUNDED_WORKSPACE (no f16 staging of a q8_0
         cache: the workspace does not grow with the cache).  ``gate`` (the layer prologue's qg,
-        f32 [S, rows, H, 2D]) sets SIXI_ATTN_FLAG_GATE: out = attention * sigmoid(qg[..., D:])."""
+        f32 [S, rows, H, 2D]) sets SIXI_ATTN_FLAG_GATE: out = attention * sigmoid(qg[..., D:]).
+        ``split_prefill`` sets SIXI_ATTN_FLAG_SPLIT_PREFILL (the workspace is this call's alone
+        while it runs; :meth:`workspace_bytes` then includes a split prefill's sums)."""
         import torch
 
         D = q.shape[-1]
@@ -353,6 +354,8 @@ class FlashAttnExt:
         p.q_len = q_len.data_ptr() if q_len is not None else None
         p.mask_mode = mask_mode
         p.flags = FLAG_BOUNDED_WORKSPACE if bounded_workspace else 0
+        if split_prefill:
+            p.flags |= FLAG_SPLIT_PREFILL
         if gate is not None:
             p.flags |= FLAG_GATE
             p.gate_qg = view_of(gate, tokens_heads=False)
@@ -386,17 +389,29 @@ class FlashAttnExt:
 
     def __call__(self, q, k, v, out, kv_len=None, q_len=None, mask_mode=MASK_BLOCK_CAUSAL, mask=None,
                  scale=None, max_bias=0.0, logit_softcap=0.0, kv_type=None, stream=None, check=True,
-                 workspace=None, noalloc=False, page_table=None, bounded_workspace=False, gate=None) -> int:
+                 workspace=None, noalloc=False, page_table=None, bounded_workspace=False, gate=None,
+                 split_prefill=None) -> int:
         """One call.  ``noalloc=True`` runs sixi_attn_forward_noalloc (the library's fixed
         device scratch, no workspace); ``page_table`` reads k and v as page pools;
         ``bounded_workspace`` never stages a q8_0 cache as f16; ``gate`` fuses the layer's
-        output gate (see :meth:`params`)."""
+        output gate (see :meth:`params`).
+
+        ``split_prefill``: whether a prompt block too short to fill the GPU may share its cells
+        among work-groups that leave sums in a workspace of the call's own (another order of the
+        sums, so results agree with the unsplit call's to rounding).  None: eager calls on the
+        current stream do, on a buffer from torch's allocator; captured ones, and those with an
+        explicit ``stream``, ``workspace`` or ``noalloc``, do not.  True: those too -- the given
+        workspace (or the fixed scratch) is this call's alone while it runs, or the capture is
+        torch.cuda.graph's, whose memory pool gives the buffer.  False: never."""
         import torch
 
         p = self.params(q, k, v, out, kv_len, q_len, mask_mode, mask, scale, max_bias, logit_softcap,
-                        kv_type, stream, page_table, bounded_workspace, gate)
+                        kv_type, stream, page_table, bounded_workspace, gate, split_prefill)
         if p.stream is None:
             p.stream = torch.cuda.current_stream(self.device).cuda_stream
+        elif split_prefill and workspace is None and not noalloc:
+            if p.stream != torch.cuda.current_stream(self.device).cuda_stream:
+                raise ValueError("a split prefill on a stream that is not torch's current one needs a workspace")
         if noalloc:
             rc = self.lib.sixi_attn_forward_noalloc(ctypes.byref(p))
             if check and rc != OK:
@@ -407,7 +422,8 @@ class FlashAttnExt:
         if rc == OK:
             if workspace is not None:
                 ws = workspace
-            elif least.value < n.value and stream is None and not torch.cuda.is_current_stream_capturing():
+            elif least.value < n.value and (split_prefill or (split_prefill is None and stream is None and
+                                                              not torch.cuda.is_current_stream_capturing())):
                 # the call's own until its kernels are queued (threads that share the stream may queue
                 # theirs in between), then the allocator's, which reuses it in this stream's order
                 ws = torch.empty(n.value, dtype=torch.uint8, device=self.device)

@@ -154,6 +154,47 @@ def test_layer_graph_fused_gate():
     assert torch.equal(out, fused)
 
 
+@pytest.mark.parametrize("kv_type", [sa.TYPE_F16, sa.TYPE_Q8_0])
+def test_short_prompt_graph(kv_type):
+    """A prompt block short enough to split, captured after one eager call on a fresh handle: by default the
+    replays equal the unsplit call and the capture leaves the handle's buffers as they were; on request
+    (the graph pool's memory, or a workspace of the caller's) they equal the eager call, which splits."""
+    w = wl.Workload("graph short prompt", 0x51A7_B700, 1, [4000], [40], kv_type=kv_type)
+    dev = wl.to_device(wl.make_host(w))
+    out = torch.empty((1, 40, w.H, w.D), device="cuda")
+    _say(f"graph: short prompt kv_type={kv_type}")
+
+    def call(fa, **kw):
+        fa(dev["q"], dev["k"], dev["v"], out, kv_len=dev["kv_len"], q_len=dev["q_len"], **kw)
+
+    def result(fa, **kw):
+        call(fa, **kw)
+        torch.cuda.synchronize()
+        return out.clone()
+
+    fa = sa.FlashAttnExt()
+    split = result(fa)
+    buffer = fa._ws
+    own = torch.empty(fa.workspace_bytes(fa.params(dev["q"], dev["k"], dev["v"], out, kv_len=dev["kv_len"],
+                                                   q_len=dev["q_len"], split_prefill=True)),
+                      dtype=torch.uint8, device="cuda")
+    whole = result(sa.FlashAttnExt(), split_prefill=False)
+    assert not torch.equal(split, whole)   # (the sums' order: the case is meant to split)
+    for want, kw in ((whole, {}), (split, {"split_prefill": True}), (split, {"split_prefill": True, "workspace": own})):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            call(fa, **kw)
+        assert fa._ws is buffer
+        for r in range(3):
+            out.zero_()
+            _ = torch.ones(1 << 22, device="cuda").sum().item()   # eager work between replays
+            assert torch.equal(result(fa), split)
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), (r, kw.keys())
+
+
 def test_gdn_graph():
     """GDN verify out of place (the input state stays fixed, so every replay has the same input);
     16 streams x 48 groups = 1536 items, more than the work-groups that fit at once, so the

@@ -107,3 +107,22 @@ def test_an_eager_split_call_sizes_what_the_captured_one_uses(handle, q8, monkey
     _call(fa, q8=q8)
     assert fa._ws is kept
     assert used == [(kept.data_ptr(), kept.numel(), 0)]
+
+
+def test_who_splits(handle):
+    """By default only eager calls on the current stream split; with split_prefill=True the others do, on
+    memory that is theirs: the caller's workspace, or (under torch's capture) its pool's."""
+    fa, state = handle
+    flags = []
+    state["launch"] = lambda p: flags.append(bool(p.flags & sa.FLAG_SPLIT_PREFILL))
+    ws = torch.empty(128 << 20, dtype=torch.uint8)
+    assert ws.data_ptr() % 64 == 0
+    for capturing in (False, True):
+        state["capturing"] = capturing
+        for split in (None, True, False):
+            _call(fa, split_prefill=split)
+            _call(fa, split_prefill=split, stream=STREAM)  # the current stream, by its handle
+            _call(fa, split_prefill=split, stream=STREAM + 8, workspace=ws)
+    assert flags == [True, False, False, True, True, True] + [False] * 3 + [False] * 3 + [True] * 3 + [False] * 3
+    with pytest.raises(ValueError):
+        _call(fa, split_prefill=True, stream=STREAM + 8)
