@@ -69,7 +69,9 @@ struct FaArgs {
     int32_t seg_cost;      // tiles' worth of work charged to each segment in the split
     int64_t slot_floats;   // floats per partial slot
     int32_t* seg_pieces;   // per segment: logical work-groups of its first and last piece
-    int32_t pf_split;      // prefill: work-groups that share the cells of each row block (>= 1)
+    int32_t pf_split;      // prefill: work-groups launched for each row block (>= 1), at most that many of
+                           // which share its cells (prefill_shares)
+    const int32_t* share_len;  // the call's kv_len, also where a mask's lengths stand in for it
     int32_t q_q8;          // prefill over an f16-staged q8_0 cache: convert Q to the q8_0 dot type
                            // in the kernel (ggml's rule), as the q8_0 kernels do
 
@@ -193,6 +195,18 @@ constexpr int kPrefillCells = 64;  // cells per tile
 constexpr int prefill_row_blocks(int64_t n_q, int G) { return (int)((n_q * G + kPrefillRows - 1) / kPrefillRows); }
 // Floats of one work-group's share of a split row block: O rows, m and l.
 constexpr int prefill_slot_floats(int head_dim) { return kPrefillRows * (head_dim + 2); }
+// Shares that walk a row block over a stream of n_cells cells where the launch has room for `split`:
+// the launch is sized for the cache, whose capacity is all the host knows, the shares for the cells in
+// use.  Two tiles are the least that pays (us, one stream in a 32768-cell cache, at least 4, 3, 2 and 1
+// tiles a share): 64 rows behind 500 cells at 256 dims 29.7, 29.8, 25.5, 25.5; behind 1000 at 256 dims
+// 31.7, 29.7, 29.0, 30.6, and at 128 dims (pages) 19.5, 17.9, 18.3, 22.2; 173 rows behind 300 cells of
+// 11776 at 256 dims 36.8, 30.9, 30.4, 30.8.  Every launched share walking, and merging, whatever the
+// length took 26.6 us for 64 rows behind no cell at all (15.3 now, of which the merge launch, which
+// finds nothing to do, is 4; 10.6 unsplit).
+constexpr int kPrefillShareCells = 2 * kPrefillCells;
+constexpr int prefill_shares(int n_cells, int split) {
+    return n_cells < 2 * kPrefillShareCells ? 1 : n_cells / kPrefillShareCells < split ? n_cells / kPrefillShareCells : split;
+}
 // Work-groups that fit a CU (LDS).
 constexpr int prefill_groups_per_cu(int head_dim) { return head_dim == 128 ? 2 : 1; }
 // Work-groups sharing each of `blocks` row blocks (1: no split).  Blocks that reach more than half

@@ -105,6 +105,15 @@ __device__ __forceinline__ f32x16 mfma32x32x16(f16x8 a, f16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
+// Work-groups that share a row block of stream s, as prefill_merge counts them.
+__device__ __forceinline__ int stream_shares(const FaArgs& a, int s) {
+    if (a.pf_split == 1) return 1;
+    FaArgs own = a;
+    own.kv_len = a.share_len;
+    own.kv_len_stride = 1;
+    return prefill_shares(stream_dims(own, s).nc, a.pf_split);
+}
+
 // QQ8: Q goes through ggml's conversion to the q8_0 dot type (a q8_0 cache, read as q8_0 tiles or
 // staged as f16 rows).
 // LEAN: the DMA offsets of the K/V tiles are worked out per tile instead of held in registers (256-dim
@@ -161,8 +170,13 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
     const int t_full = (MODE == MODE_GENERIC) ? 0 : vis_min / kBN;
     constexpr bool RAW = MODE != MODE_GENERIC;  // scores in raw dot-product units
     // the tiles walked: all of them, or (split) this work-group's share
-    const int t_beg = (int)((int64_t)n_tiles * chunk / a.pf_split);
-    const int t_end = (int)((int64_t)n_tiles * (chunk + 1) / a.pf_split);
+    const int n_shares = stream_shares(a, s);
+    if (chunk >= n_shares) return;
+    // (one scalar register across the tile loop for the two)
+    int piece = chunk | n_shares << 8;
+    asm volatile("" : "+s"(piece));
+    const int t_beg = (int)((int64_t)n_tiles * chunk / n_shares);
+    const int t_end = (int)((int64_t)n_tiles * (chunk + 1) / n_shares);
 
     // ---- Q^T B operands in registers: lane l -> row j, dims 16ks + 8*hl .. +7 ----
     // (every load issued before any is used; rows past the block read its first row)
@@ -708,19 +722,20 @@ __device__ __forceinline__ void prefill_body(const FaArgs& a, int causal, int nr
         auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_sum), __float_as_uint(l_sum), false, false);
         l_sum = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
     }
-    // (the row and its address are recomputed from the lane here rather than held across the
-    // tile loop)
-    int lx = lane;
-    asm volatile("" : "+v"(lx));
+    // (the row and its address are worked out anew from the lane here rather than held across the
+    // tile loop, as is the divisor's reciprocal)
+    int lx = lane, G = a.G;
+    asm volatile("" : "+v"(lx), "+s"(G));
     const int hw = lx >> 5;
     const int rw = 32 * wq + (lx & 31);  // row in the group
+    const int ch = piece & 255, shares = piece >> 8;
     if (r0 + rw < n_rows) {
-        const bool share = a.pf_split > 1;  // a split item's share: plain sums, and their exponent reference (log2 units)
-        const int jw = (r0 + rw) / a.G, hd = g * a.G + (r0 + rw) % a.G;
+        const bool share = shares > 1;  // a split item's share: plain sums, and their exponent reference (log2 units)
+        const int jw = (r0 + rw) / G, hd = g * G + (r0 + rw) % G;
         float inv = l_sum == 0.0f ? 0.0f : 1.0f / l_sum;
         char* dst = a.out + (int64_t)jw * a.o_nb2 + (int64_t)hd * a.o_nb1 + (int64_t)s * a.o_nb3;
         if (share) {
-            float* slot = a.part + (int64_t)(chunk + a.pf_split * (g + a.Hkv * (s + a.S * rb))) * PrefillSlot<D>::FLOATS;
+            float* const slot = a.part + (int64_t)(ch + a.pf_split * (g + a.Hkv * (s + a.S * rb))) * PrefillSlot<D>::FLOATS;
             if (hw == 0) {
                 // (no reference yet: -inf if the share saw no cell of the row, else -- c2 = 0, whose
                 // threshold nothing exceeds -- the 0 that its probabilities were taken against)
@@ -757,21 +772,23 @@ __global__ __launch_bounds__(kThreads) void prefill_merge(FaArgs a) {
     const int r = rb * kBM + rw;
     if (r >= sd.ql * a.G) return;
     const float* slot = a.part + (int64_t)item * a.pf_split * PrefillSlot<D>::FLOATS;
+    const int n_shares = prefill_shares(sd.nc, a.pf_split);
+    if (n_shares == 1) return;  // written by the work-group that walked the whole block
     float m = neg_inf(), l = 0.0f;
     f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int c0 = 0; c0 < a.pf_split; c0 += kU) {
+    for (int c0 = 0; c0 < n_shares; c0 += kU) {
         float mc[kU], lc[kU];
         f32x4 oc[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const float* p = slot + (int64_t)min(c0 + u, a.pf_split - 1) * PrefillSlot<D>::FLOATS;
+            const float* p = slot + (int64_t)min(c0 + u, n_shares - 1) * PrefillSlot<D>::FLOATS;
             mc[u] = p[PrefillSlot<D>::M + rw];
             lc[u] = p[PrefillSlot<D>::L + rw];
             oc[u] = *reinterpret_cast<const f32x4*>(p + rw * D + d);
         }
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            if (c0 + u >= a.pf_split) break;
+            if (c0 + u >= n_shares) break;
             const float mn = fmaxf(m, mc[u]);
             // (equal references, both -inf among them, keep their sums as they are)
             const float wo = m == mn ? 1.0f : fast_exp2(m - mn), wn = mc[u] == mn ? 1.0f : fast_exp2(mc[u] - mn);

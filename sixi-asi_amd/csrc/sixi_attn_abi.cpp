@@ -258,7 +258,7 @@ int resolve(const sixi_attn_params* p, Plan* out, size_t stage_cap = SIXI_ATTN_S
     }
     a.out = static_cast<char*>(const_cast<void*>(o.data));
     a.o_nb1 = o.nb[1]; a.o_nb2 = o.nb[2]; a.o_nb3 = o.nb[3];
-    a.kv_len = p->kv_len;
+    a.kv_len = a.share_len = p->kv_len;
     a.kv_len_stride = 1;
     a.q_len = p->q_len;
     if (mode == SIXI_MASK_EXPLICIT) {

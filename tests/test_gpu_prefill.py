@@ -158,15 +158,20 @@ def test_prefill_f16_queries(fa):
         _check(want[s, :w.q_len[s]], got[s, :w.q_len[s]], f"f16 Q stream {s}")
 
 
-def _forward(fa, p, split, ws=None):
-    """sixi_attn_forward of `p` with or without the split, on a workspace of its own full of NaN bits."""
+def _sizes(fa, p):
     least, full = ctypes.c_size_t(0), ctypes.c_size_t(0)
     assert fa.lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(full)) == sa.OK
     assert least.value < full.value, "the case is meant to split"
+    return least.value, full.value
+
+
+def _forward(fa, p, split, ws=None):
+    """sixi_attn_forward of `p` with or without the split, on a workspace of its own full of NaN bits."""
+    least, full = _sizes(fa, p)
     if split:
         p.flags |= sa.FLAG_SPLIT_PREFILL
     if ws is None:
-        ws = torch.full((full.value if split else least.value,), 0xFF, dtype=torch.uint8, device="cuda")
+        ws = torch.full((full if split else least,), 0xFF, dtype=torch.uint8, device="cuda")
     p.stream = torch.cuda.current_stream().cuda_stream
     p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
     rc = fa.lib.sixi_attn_forward(ctypes.byref(p))
@@ -292,3 +297,40 @@ def test_split_in_the_fixed_scratch(fa):
             assert same == (fits or not split)
             for s in range(w.S):
                 _check(want[s, :q_len[s]], outs[0][s, :q_len[s]], f"stream {s} split={split}")
+
+
+@pytest.mark.parametrize("D", [128, 256])
+@pytest.mark.parametrize("cached", [0, 87, 216, 3000])
+def test_shares_follow_the_cells_in_use(fa, cached, D):
+    """A split launch is sized for the cache (16384 cells, NaN past the stream's); the cells in use decide
+    how many work-groups share them, at least 128 cells each (40 rows behind 216 cells: two shares), and
+    the others write nothing.  With one share the sums are left alone and the output is the unsplit
+    call's bit for bit; always against the oracle."""
+    _say(f"short stream in a long cache: cached={cached} D={D}")
+    w = wl.Workload("short stream", 0x51A7_5500 + cached + D, 1, [cached], [40], D=D)
+    host = wl.make_host(w)
+    dev = wl.to_device(host)
+    k, v = (torch.full((1, 16384, w.Hkv, D), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+    for x, c in ((k, dev["k"]), (v, dev["v"])):
+        x[:, :cached + 40] = c.view(torch.float16)[:, :cached + 40]
+    outs = []
+    for split in (True, False):
+        out = torch.full((1, 40, w.H, D), float("nan"), dtype=torch.float32, device="cuda")
+        p = fa.params(dev["q"], k, v, out, kv_len=dev["kv_len"], q_len=dev["q_len"])
+        least, full = _sizes(fa, p)
+        ws = torch.full((full if split else least,), 0xA5, dtype=torch.uint8, device="cuda")
+        _forward(fa, p, split, ws)
+        outs.append(out.cpu().numpy())
+        if split:
+            blocks, slot = 4 * 2, 128 * (D + 2) * 4   # kv-heads x row blocks of 40 x 6 rows; bytes of a share
+            launched = (full - least) // (blocks * slot)
+            sums = ws[least:least + blocks * launched * slot].view(blocks, launched, slot)
+            shares = max(1, min(launched, (cached + 40) // 128))
+            assert launched > 2 and shares == {0: 1, 87: 1, 216: 2, 3000: launched}[cached]
+            assert bool(torch.all(sums[:, shares if shares > 1 else 0:] == 0xA5))
+            if shares > 1:
+                assert not bool(torch.any(torch.all(sums[:, :shares] == 0xA5, dim=-1)))
+    if cached < 216:
+        assert np.array_equal(outs[0], outs[1])
+    want = oracle.attention_for_workload(host, w.kv_type)
+    _check(want, outs[0], "split")
