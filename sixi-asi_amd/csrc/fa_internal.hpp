@@ -209,30 +209,35 @@ constexpr int prefill_shares(int n_cells, int split) {
 }
 // Work-groups that fit a CU (LDS).
 constexpr int prefill_groups_per_cu(int head_dim) { return head_dim == 128 ? 2 : 1; }
-// Work-groups sharing each of `blocks` row blocks (1: no split).  Blocks that reach more than half
+// Work-groups launched for each of `blocks` row blocks (1: no split).  Blocks that reach more than half
 // of the CUs are left whole: what idle CUs could take off them is then near what the sums' way
-// through memory costs.  A share walks n / C tiles and costs kStart tiles of start-up (Q, the
-// first tile, the sums' way out); its sums cross memory twice (kMerge tiles' time over the whole
-// chip).  Every C up to 16 whose launch stays within two full rounds is priced by its rounds; n_kv
-// stands in for the lengths, which only the device knows.  Measured at one share and more (us, the
-// last one is what the rule takes):
-//   1 x 173 rows behind 11400 cells, 256 dims f16   1: 552   4: 157   6: 114   7: 101
-//   4 x 40 rows behind 12000 cells, 256 dims        1: 577   4: 164   6: 118   8: 97
-//   1 x 300 rows behind 20000 cells, 128 dims       1: 413   4: 118   6: 108   8: 97
-//   1 x 64 rows behind 4000 cells, 128 dims         1: 87    4: 32    8: 24.8  10: 25.4
-//   1 x 600 rows behind 2000 cells, 256 dims        1: 132   2: 88
-//   1 x 17 rows behind 300 cells, 128 dims          1: 12.9  2: 13.2
+// through memory costs.  A share walks ceil(n / C) tiles and costs kStart tiles of start-up (Q, the
+// first tile, the sums' way out); a split costs the merge's launch (kSplit tiles' time) and its
+// sums cross memory twice (kMerge tiles' time over the whole chip).  Every C up to 16 whose launch
+// stays within two full rounds is priced by its rounds; n_kv stands in for the lengths, which only
+// the device knows.  Measured (us of GPU time at C, the last one is what the rule takes):
+//   1 x 173 rows behind 11400 cells, 256 dims f16   1: 553   4: 164   6: 122   8: 169   7: 111
+//   4 x 40 rows behind 12000 cells, 256 dims        1: 580   4: 169   6: 125   9: 165   8: 106
+//   1 x 300 rows behind 20000 cells, 128 dims       1: 415   4: 128   6: 125   16: 122  8: 111
+//   1 x 64 rows behind 4000 cells, 256 dims         1: 202   8: 45.6  10: 44.4 16: 39.7 13: 38.9
+//   1 x 64 rows behind 4000 cells, 128 dims         1: 87.6  4: 32.1  8: 25.0  16: 27.8 13: 25.7
+//   1 x 600 rows behind 2000 cells, 256 dims        1: 139   3: 111   4: 105   2: 94
+//   1 x 600 rows behind 2000 cells, 128 dims        1: 63.3  2: 46.2  3: 43.7  8: 56.1  4: 41.2
+//   1 x 17 rows behind 2000 cells, 128 dims         1: 46.3  4: 20.5  8: 17.1  9: 17.1
+//   1 x 17 rows behind 300 cells, 128 dims          2: 12.9  1: 12.0
+//   1 x 200 rows behind 500 cells, 256 dims         1: 44.1  2: 35.7  3: 37.4
+//   1 x 400 rows behind 600 cells, 128 dims         4: 28.3  3: 26.3  2: 25.8  1: 28.2
 inline int prefill_split(int64_t blocks, int64_t n_kv, int head_dim, int cu_count) {
     if (2 * blocks > cu_count) return 1;
-    constexpr double kStart = 4.0;
-    const double kMerge = 0.05;
+    constexpr double kStart = 4.0, kSplit = 4.0, kMerge = 0.03;
     const int64_t slots = (int64_t)cu_count * prefill_groups_per_cu(head_dim);
     const int64_t tiles = (n_kv + kPrefillCells - 1) / kPrefillCells;
     int best = 1;
     double best_cost = 0.0;
     for (int c = 1; c <= 16 && (c == 1 || blocks * c <= 2 * slots) && (c == 1 || tiles >= 4 * c); ++c) {
         const int64_t rounds = (blocks * c + slots - 1) / slots;
-        const double cost = (double)rounds * ((double)tiles / c + kStart) + (c > 1 ? kMerge * (double)(blocks * c) : 0.0);
+        const double cost = (double)rounds * ((double)((tiles + c - 1) / c) + kStart) +
+                            (c > 1 ? kSplit + kMerge * (double)(blocks * c) : 0.0);
         if (c == 1 || cost < best_cost) {
             best = c;
             best_cost = cost;

@@ -242,6 +242,23 @@ def test_prefill_sums_only_on_request():
         assert least.value == full.value
 
 
+@pytest.mark.parametrize("rows,n_kv,D,want", [
+    (17, 512, 128, 1),       # the merge's launch costs more than the second work-group saves (12.9 against 12.0 us)
+    (64, 4096, 256, 13),     # few blocks: many shares (38.9 us; ten took 44.4)
+    (173, 11776, 256, 7),    # one round of the 256 CUs (110.6; eight take two rounds, 168.8)
+    (600, 2816, 128, 4),     # one round of two work-groups a CU (41.2; three took 43.7)
+    (700, 4096, 128, 1),     # blocks on more than half of the CUs
+])
+def test_prefill_shares(rows, n_kv, D, want):
+    """Work-groups launched per row block, as the workspace names them (256 CUs: also where no GPU is)."""
+    lib = sa.load_library()
+    p = _params(S=1, n_q=rows, n_kv=n_kv, D=D)
+    least, full = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    assert lib.sixi_attn_workspace_range(ctypes.byref(p), ctypes.byref(least), ctypes.byref(full)) == sa.OK
+    share = 4 * -(-rows * 6 // 128) * 128 * (D + 2) * 4
+    assert (full.value - least.value) // share == (want if want > 1 else 0)
+
+
 def _paged_params(S, stride, n_q=1, n_pages=1024):
     """A paged call: K and V pools of 256-cell pages, a page table of `stride` pages per stream."""
     p = _params(S=S, n_q=n_q)
