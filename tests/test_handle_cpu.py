@@ -137,3 +137,21 @@ def test_a_bounded_workspace_stays_a_token(handle, q8):
     for n_kv in (1024, 4096, 32768):
         _call(fa, n_kv=n_kv, q8=q8, bounded_workspace=True)
     assert max(sizes) <= 4096 and _held(fa) <= 4096
+
+
+def test_views_hold_what_they_are_given():
+    """The packed view against the fields one by one: Python and numpy integers, a null pointer, the
+    extents and strides of permuted and sliced tensors."""
+    import numpy as np
+
+    for ptr, ne, nb in ((0x7F12_3456_7890, [1, 2, 3, 4], [4, 8, 16, 32]),
+                        (None, np.array([1 << 40, 5, 0, -1]), [np.int32(2), -16, 1 << 62, 0])):
+        v = sa.make_view(ptr, sa.TYPE_F16, ne, nb)
+        assert v.data == ptr and v.type == sa.TYPE_F16 and v.reserved == 0
+        assert list(v.ne) == [int(x) for x in ne] and list(v.nb) == [int(x) for x in nb]
+    t = torch.zeros((3, 5, 7, 64), dtype=torch.float16).permute(0, 2, 1, 3)[:, 1:, ::2]
+    v = sa.view_of(t)
+    assert v.data == t.data_ptr() and list(v.ne) == [64, 6, 3, 3]
+    assert list(v.nb) == [2, 64 * 2, 2 * 7 * 64 * 2, 5 * 7 * 64 * 2]
+    v = sa.view_of(t, tokens_heads=False)
+    assert list(v.ne) == [64, 3, 6, 3] and list(v.nb) == [2, 2 * 7 * 64 * 2, 64 * 2, 5 * 7 * 64 * 2]
