@@ -14,6 +14,7 @@ no CPU fallback: a missing library raises ``SixiAttnUnavailable``.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import os
 import pathlib
@@ -286,6 +287,13 @@ def make_view(data_ptr: int, type_id: int, ne, nb) -> SixiView:
                                                 int(nb[0]), int(nb[1]), int(nb[2]), int(nb[3])))
 
 
+@functools.lru_cache(maxsize=None)
+def _float_types() -> dict:
+    import torch
+
+    return {torch.float32: TYPE_F32, torch.float16: TYPE_F16}
+
+
 def view_of(t, type_id: Optional[int] = None, head_dim: Optional[int] = None,
             tokens_heads: bool = True) -> SixiView:
     """ggml view of a 4-d torch tensor whose last dim is innermost.
@@ -294,8 +302,6 @@ def view_of(t, type_id: Optional[int] = None, head_dim: Optional[int] = None,
     (Q, K, V as llama.cpp permutes them); False: the plain reversal (out, mask).
     For q8_0 pass a uint8 tensor whose last dim holds the packed blocks and ``head_dim``.
     """
-    import torch
-
     if t.dim() != 4:
         raise ValueError("expected a 4-d tensor")
     es = t.element_size()
@@ -304,8 +310,10 @@ def view_of(t, type_id: Optional[int] = None, head_dim: Optional[int] = None,
     nb = [strides[i] * es for i in order]
     ne = [shape[i] for i in order]
     if type_id is None:
-        type_id = {torch.float32: TYPE_F32, torch.float16: TYPE_F16}[t.dtype]
+        type_id = _float_types()[t.dtype]
     if type_id == TYPE_Q8_0:
+        import torch
+
         if t.dtype != torch.uint8 or head_dim is None or t.shape[-1] != head_dim // 32 * 34:
             raise ValueError("q8_0 view needs a uint8 tensor of D/32*34 bytes per row and head_dim")
         if t.stride(-1) != 1:
