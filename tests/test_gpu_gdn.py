@@ -78,6 +78,12 @@ def test_reference_kernel_test_case():
     assert np.array_equal(y1, y2) and np.array_equal(s1, s2)        # bitwise repeatable
 
 
+# 128-dim keys run one of two kernels: up to 64 states of 128 rows (128 of 64) the one whose work-groups
+# of 32 state rows fit the 256 CUs at once, beyond that the one with 64 rows per work-group.  (streams,
+# groups) on either side of the line:
+BOTH_KERNELS = pytest.mark.parametrize("S,G", [(2, 6), (12, 6)])
+
+
 @pytest.mark.parametrize("decay_first", [False, True])
 def test_qwen_verify_block(decay_first):
     # 48 value heads of 128 with 128-dim keys (ssm_time_step_rank 48, ssm_state_size 128), 16 rows
@@ -92,9 +98,21 @@ def test_other_shapes_out_of_place(K, HD):
     _run(*args, q_len=[5, 2, 4], in_place=False, label=f"K={K} HD={HD}")
 
 
-def test_long_block_several_staging_passes():
-    args = _inputs(2, 40, 4, 128, 128, 31)                           # 16 + 16 + 8 rows
-    _run(*args, q_len=[40, 33], snap=[17, 33], label="40 rows")
+@pytest.mark.parametrize("S,G", [(2, 4), (12, 6)])
+def test_long_block_several_staging_passes(S, G):
+    args = _inputs(S, 40, G, 128, 128, 31)                           # 16 + 16 + 8 rows
+    _run(*args, q_len=[40, 33] * (S // 2), snap=[17, 33, 40, 16][:S] * max(1, S // 4), label="40 rows")
+
+
+@pytest.mark.parametrize("decay_first", [False, True])
+@pytest.mark.parametrize("S,G", [(3, 7), (12, 11)])
+def test_64_row_states_of_128_dim_keys(S, G, decay_first):
+    # 42 work-groups of 32 state rows, and 264: one more than a multiple of 8 states over the line
+    n = 40
+    q_len = [40, 17, 33, 0, 16, 1, 32, 40, 15, 39, 31, 2][:S]
+    snap = [39, 17, 16, 0, 3, 0, 32, 1, 15, 17, 30, 2][:S]
+    _run(*_inputs(S, n, G, 128, 64, 91 + S), q_len=q_len, snap=snap, decay_first=decay_first,
+         in_place=decay_first, label="64-row states")
 
 
 @pytest.mark.parametrize("decay_first", [False, True])
@@ -113,12 +131,14 @@ def test_several_items_per_work_group(decay_first):
     _run(*args, q_len=q_len, snap=snap, decay_first=decay_first, label="3072 items")
 
 
-def test_strided_views():
+@pytest.mark.parametrize("S,G", [(16, 48), (3, 20)])
+def test_strided_views(S, G):
     # ggml views that are not packed: q and k stored group-major ([S][G][n][K] seen as [S][n][G][K]),
     # v, y and both states in padded rows, alpha and beta every other float; out of place, so the
     # padding of y and of the output state must stay untouched; 16 streams x 48 groups = 1536 items
-    # (several per work-group, the XCD pairing on), blocks of up to 20 rows
-    S, n, G, K, HD = 16, 20, 48, 128, 128
+    # (several per work-group, the XCD pairing on), and 60 states in one round of work-groups of 32
+    # state rows; blocks of up to 20 rows
+    n, K, HD = 20, 128, 128
     q, k, v, al, be, S0 = _inputs(S, n, G, K, HD, 81)
     rng = np.random.default_rng(82)
     q_len = [int(x) for x in rng.integers(0, n + 1, S)]
@@ -164,30 +184,32 @@ def test_no_lengths():
     _run(*_inputs(2, 3, 3, 128, 128, 41), label="no lengths")
 
 
-def test_extreme_gates():
+@BOTH_KERNELS
+def test_extreme_gates(S, G):
     # alpha 0 resets the state to the row's write, alpha 1 keeps it; beta 0 writes nothing, beta 1
     # writes the whole correction
-    q, k, v, al, be, S0 = _inputs(2, 8, 6, 128, 128, 51)
+    q, k, v, al, be, S0 = _inputs(S, 8, G, 128, 128, 51)
     al[:, ::2] = 0.0
     al[:, 1::4] = 1.0
     be[:, :, ::3] = 0.0
     be[:, :, 1::3] = 1.0
-    _run(q, k, v, al, be, S0, q_len=[8, 5], snap=[8, 4], label="alpha 0/1, beta 0/1")
+    _run(q, k, v, al, be, S0, q_len=[8, 5] * (S // 2), snap=[8, 4] * (S // 2), label="alpha 0/1, beta 0/1")
 
 
 @pytest.mark.parametrize("decay_first", [False, True])
-def test_decays_that_leave_the_carried_scale_range(decay_first):
+@pytest.mark.parametrize("G", [6, 18])   # 24 states, and 72: one kernel each
+def test_decays_that_leave_the_carried_scale_range(G, decay_first):
     # the kernel carries the state as a scalar times a matrix and folds the scalar in when the
     # running product of the gates leaves [2^-30, 2^30]: gates of 2^-20 (the product leaves the range
     # at the second), 2^-40 (at once), 0 (a reset) and 4 (growth, the product passes 2^30 at the
     # 16th row), across staging passes, against the oracle's step by step recurrence
-    q, k, v, al, be, S0 = _inputs(4, 40, 6, 128, 128, 61)
+    q, k, v, al, be, S0 = _inputs(4, 40, G, 128, 128, 61)
     al[0, 3:6] = 2.0 ** -20
     al[1, 10] = 2.0 ** -40
     al[1, 20] = 0.0
     al[2, :] = 4.0
     al[3, 14:18] = 2.0 ** -20
-    S, n, G, K = q.shape
+    S, n, _, K = q.shape
     d = [torch.from_numpy(x).cuda() for x in (q, k, v, al, be)]
     st = torch.from_numpy(S0).cuda()
     y = torch.full((S, n, G, 128), float("nan"), dtype=torch.float32, device="cuda")
