@@ -48,6 +48,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "device_util.hpp"
 #include "gdn_internal.hpp"
 
 namespace sixi {
@@ -528,9 +529,9 @@ __global__ __launch_bounds__(256) void gdn_verify_chunked_kernel(GdnArgs a, int 
 //     the same with q and k q^T.  First half: wave 4 makes L and wave 6 makes W of chunk i + 2,
 //     wave 7 stages v, the gates and their products E of chunk i + 3, wave 5 inverts I + L of chunk
 //     i + 1.  Each issues the global loads of its chunk two iterations ahead.
-// Every SIMD holds one consumer and one producer, whose 56 and 16 f32 MFMAs (32 cycles each) per
-// iteration are its floor: 2304 cycles, 123 us over the 128 chunks of 2048 rows, which take 307 us
-// (a call; 739 with the chunked kernel).  Before each producer wave had a loop of its own it took 325
+// Every SIMD holds one consumer and one producer, whose 56 and 16 f32 MFMAs (32 cycles each; wave 5's
+// 32, with the inverse) per iteration are its floor: 2816 cycles on the busiest SIMD, 150 us over the 128
+// chunks of 2048 rows, which take 307 us (a call; 739 with the chunked kernel).  Before each producer wave had a loop of its own it took 325
 // in graph replays, of which the producers switched off left 219 (the consumers' chain P -> exchange
 // -> U -> state); the inversion was 35 of it, the staging loads 28, E 27, k k^T and k q^T 24.
 constexpr int kScanRows = 32;
@@ -876,16 +877,6 @@ hipError_t launch_chunked_df(const GdnArgs& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-int cu_count() {
-    static int cached = -1;
-    if (cached < 0) {
-        int dev = 0, n = 0;
-        cached = hipGetDevice(&dev) == hipSuccess &&
-                 hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? n : 0;
-    }
-    return cached;
-}
-
 template <int HD>
 hipError_t launch_scan(const GdnArgs& a, hipStream_t stream) {
     const int64_t groups = (int64_t)a.S * a.G * (HD / kScanRows);
@@ -900,10 +891,13 @@ hipError_t launch_scan(const GdnArgs& a, hipStream_t stream) {
 template <int HD>
 hipError_t launch_chunked(const GdnArgs& a, hipStream_t stream) {
     // While its work-groups fit the CUs at once the scan kernel is the faster one at every length (48
-    // groups, one stream: 4 rows 9.4 -> 8.7 us, 16 rows 9.6 -> 9.0, 33 rows 18.1 -> 15.0, 2048 rows
-    // 674 -> 325); beyond that its eight waves per CU lose to the sixteen of the chunked kernel (two
-    // streams, an earlier form of it: 16 rows 10.1 against 15.0 us, 128 rows 46 against 55).
-    if ((int64_t)a.S * a.G * (HD / kScanRows) <= cu_count()) return launch_scan<HD>(a, stream);
+    // groups of 128 rows, one stream, graph replays: 4 rows 9.2 -> 8.0 us, 16 rows 9.4 -> 8.2, 128 rows
+    // 40.8 -> 27.5, 2048 rows 674 -> 295); beyond that its eight waves per CU lose to the sixteen of the
+    // chunked kernel (chunked against scan: two streams, 16 rows 10.0 against 14.1, 128 rows 45.0 against
+    // 51.7; four streams, 128 rows 61.9 against 77.7, 1024 rows 473 each; eight streams, 512 rows 311 against
+    // 493).  Long blocks of exactly two streams are the exception that the line leaves out: 512 rows
+    // 173 against 158, 2048 rows 748 against 612.
+    if ((int64_t)a.S * a.G * (HD / kScanRows) <= device_cu_count()) return launch_scan<HD>(a, stream);
     return a.decay_first ? launch_chunked_df<HD, true>(a, stream) : launch_chunked_df<HD, false>(a, stream);
 }
 

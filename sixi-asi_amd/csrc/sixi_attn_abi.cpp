@@ -15,6 +15,7 @@
 #include <mutex>
 
 #include "abi_util.hpp"
+#include "device_util.hpp"
 #include "fa_internal.hpp"
 #include "sixi_attn.h"
 
@@ -106,19 +107,6 @@ void prepass_layout(Plan& pl) {
 // Fewer shares per row block until the workspace fits in `bytes` (down to one: no split).
 void prefill_fit(Plan& pl, size_t bytes) {
     while (!pl.splitk && pl.a.pf_split > 1 && pl.ws_bytes > bytes) prefill_layout(pl, pl.a.pf_split - 1);
-}
-
-int cu_count_cached() {
-    static int cached = -1;
-    if (cached < 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            cached = n;
-        else
-            cached = 256;
-    }
-    return cached;
 }
 
 // Split-K workspace after the staging area: `slots` partial slots, then the (first, last)
@@ -379,7 +367,7 @@ int resolve(const sixi_attn_params* p, Plan* out, size_t stage_cap = SIXI_ATTN_S
         if (S * H * ((n_q + 127) / 128) > (int64_t)INT32_MAX) return SIXI_E_UNSUPPORTED;
         const int64_t blocks = S * Hkv * sixi::prefill_row_blocks(n_q, a.G);
         const bool may_split = (p->flags & SIXI_ATTN_FLAG_SPLIT_PREFILL) != 0;
-        prefill_layout(pl, may_split ? sixi::prefill_split(blocks, n_kv, pl.D, cu_count_cached()) : 1);
+        prefill_layout(pl, may_split ? sixi::prefill_split(blocks, n_kv, pl.D, sixi::device_cu_count()) : 1);
     }
     if (pl.splitk) {
         prepass_layout(pl);
@@ -415,9 +403,9 @@ char* scratch_base() {
 
 // Work-groups of the launch: the split-K grid, or (prefill) the CU count its order needs.
 int launch_groups(const Plan& pl) {
-    return pl.splitk ? sixi::decode_num_groups(pl.a, cu_count_cached(),
+    return pl.splitk ? sixi::decode_num_groups(pl.a, sixi::device_cu_count(),
                                                sixi::decode_groups_per_cu(pl.kv_type, pl.row_tiles, pl.D, pl.generic))
-                     : cu_count_cached();
+                     : sixi::device_cu_count();
 }
 
 // Launches a resolved call on `ws` (laid out as pl says).
