@@ -42,6 +42,9 @@ CASES = [
     ("decode f16 256-dim", sa.TYPE_F16, 256, [4100], [1], 24, 4, False),
     ("prefill", sa.TYPE_F16, 128, [200, 700], [150, 260], 24, 4, False),
     ("prefill 256-dim", sa.TYPE_F16, 256, [300], [130], 24, 4, False),
+    ("short prompt, split", sa.TYPE_F16, 128, [2500], [40], 24, 4, False),
+    ("short prompt 256-dim q8_0, split", sa.TYPE_Q8_0, 256, [2500, 300], [40, 20], 24, 4, False),
+    ("short prompt with the llama mask, split", sa.TYPE_F16, 128, [2500], [40], 24, 4, True),
     ("verify with the llama mask", sa.TYPE_F16, 128, [900, 5000, 37], [16, 16, 9], 24, 4, True),
     ("decode with the llama mask", sa.TYPE_F16, 128, [4096], [1], 24, 4, True),
     ("prefill with the llama mask", sa.TYPE_F16, 128, [200, 700], [150, 260], 24, 4, True),

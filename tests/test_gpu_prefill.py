@@ -21,6 +21,11 @@ pytestmark = pytest.mark.gpu
 
 MAX_ABS = 2e-3
 REL_L2 = 1e-3
+# split against unsplit: each side rounds the probabilities to f16 against other exponent references, an
+# error of 2^-10 / sqrt(12) / m for significands m, 2.07e-4 rms over log-uniform ones, independent over the
+# cells and of the other side's: sqrt(2) times that, 2.93e-4, of the sums (whose f32 order adds 1e-7); a
+# third for the spread of few rows
+SPLIT_REL_L2 = 3.9e-4
 
 
 def _say(msg):
@@ -203,50 +208,99 @@ def test_prefill_writes_no_workspace_unless_asked(fa, D):
     assert torch.equal(out, out2)
 
 
+def _paged(x):
+    """A contiguous cache [S, cells, heads, row] as a pool of shuffled 256-cell pages, and its table."""
+    S, n = x.shape[0], x.shape[1] // 256
+    order = torch.randperm(S * n, generator=torch.Generator().manual_seed(5)).cuda()
+    pages = x[:, :n * 256].reshape(S * n, 256, *x.shape[2:])
+    pool = torch.empty_like(pages)
+    pool[order] = pages
+    return pool, order.to(torch.int32).view(S, n)
+
+
 @pytest.mark.parametrize("kv_len,q_len,H,Hkv,D,kv,mode", [
-    ([1500], [17], 24, 4, 128, sa.TYPE_F16, "lengths"),         # 102 rows: one row block, 6 of them empty
-    ([700, 0, 5], [22, 17, 0], 24, 4, 256, sa.TYPE_F16, "lengths"),  # a second block of 4 rows; shares with no cell
+    ([1500], [17], 24, 4, 128, sa.TYPE_F16, "lengths"),         # 102 rows: one row block, 26 of its rows empty
+    ([700, 0, 5], [22, 17, 0], 24, 4, 256, sa.TYPE_F16, "lengths"),  # a second block of 4 rows; one share of one tile
     ([4100], [65], 8, 2, 128, sa.TYPE_Q8_0, "lengths"),         # three blocks, 66 tiles, q8_0
     ([3000, 900], [33, 20], 24, 4, 256, sa.TYPE_Q8_0, "lengths"),
+    ([17500], [20], 24, 4, 128, sa.TYPE_F16, "paged"),           # 69 pages: shares that start past the first 64
+    ([3000, 900], [33, 20], 24, 4, 256, sa.TYPE_Q8_0, "paged"),
     ([2000, 30], [40, 31], 24, 4, 128, sa.TYPE_F16, "causal"),    # the causal mask, handed over
-    ([2000, 30], [40, 31], 24, 4, 256, sa.TYPE_F16, "holes"),     # a mask with holes: the staged-mask body
+    ([2000, 30], [40, 31], 24, 4, 256, sa.TYPE_F16, "causal"),
+    ([2000, 300], [40, 31], 24, 4, 256, sa.TYPE_F16, "holes"),    # a mask with holes: the staged-mask body
+    ([2000, 300], [40, 31], 24, 4, 128, sa.TYPE_Q8_0, "holes"),
     ([1100], [24], 24, 4, 128, sa.TYPE_F16, "softcap"),          # the per-cell body
+    ([1100, 600], [24, 20], 24, 4, 256, sa.TYPE_F16, "alibi"),
 ])
 def test_split_row_blocks(fa, kv_len, q_len, H, Hkv, D, kv, mode):
-    """Few row blocks over a long cache: several work-groups share the cells of each.  Against the
-    oracle (the bar above), and against the same call without the flag (no split): the two
-    differ by the order of f32 sums and the exponent references the f16 probabilities were taken
-    against, 2^-11 of rounding each, averaged over the cells: a tenth of the bar's rel-L2 more."""
+    """Few row blocks over a long cache: several work-groups share the cells of each.  Every stream and head
+    against the oracle (the bar above); bit for bit the same when called again; and against the call
+    without the split (SPLIT_REL_L2)."""
     _say(f"split kv_len={kv_len} q_len={q_len} H={H} Hkv={Hkv} D={D} kv={kv} {mode}")
     w = wl.Workload("split_prefill", 0x51A7_5100 + sum(q_len) + D, len(kv_len), kv_len, q_len, H=H, Hkv=Hkv, D=D, kv_type=kv)
     host = wl.make_host(w, poison=True)
     dev = wl.to_device(host)
     kw = dict(kv_len=dev["kv_len"], q_len=dev["q_len"])
-    n_kv = dev["k"].shape[1]
-    if mode in ("causal", "holes"):
-        last = torch.tensor(kv_len)[:, None, None] + torch.arange(w.n_q)[None, :, None]
-        seen = torch.arange(n_kv)[None, None] <= last
-        if mode == "holes":
-            seen &= (torch.arange(n_kv) % 7 != 3)[None, None]
-        mask = torch.where(seen, 0.0, float("-inf")).to(torch.float16)[:, None].contiguous().cuda()
-        kw.update(mask_mode=sa.MASK_EXPLICIT, mask=mask)
-    if mode == "softcap":
-        kw.update(logit_softcap=20.0)
+    k, v, n_kv = dev["k"], dev["v"], dev["k"].shape[1]
+    if mode == "paged":
+        (k, kw["page_table"]), (v, _) = _paged(k), _paged(v)
+    last = np.array(kv_len)[:, None, None] + np.arange(w.n_q)[None, :, None]
+    cells = np.arange(n_kv)[None, None]
+    seen = (cells <= last) & (np.arange(w.n_q)[None, :, None] < np.array(q_len)[:, None, None])
+    if mode == "holes":
+        seen &= cells % 7 != 3
+    mask = np.where(seen, -0.02 * (last - cells) if mode == "alibi" else 0.0, -np.inf).astype(np.float16)[:, None]
+    cap = 20.0 if mode == "softcap" else 0.0
+    bias = 8.0 if mode == "alibi" else 0.0
+    if mode in ("causal", "holes", "alibi"):
+        kw.update(mask_mode=sa.MASK_EXPLICIT, mask=torch.from_numpy(mask).cuda())
+    kw.update(logit_softcap=cap, max_bias=bias)
     outs = []
-    for split in (True, False):
+    for split in (True, False, True):
         out = torch.full((w.S, w.n_q, w.H, w.D), float("nan"), dtype=torch.float32, device="cuda")
-        p = fa.params(dev["q"], dev["k"], dev["v"], out, **kw)
-        _forward(fa, p, split)
+        _forward(fa, fa.params(dev["q"], k, v, out, **kw), split)
         outs.append(out.cpu().numpy())
-    got, whole = (np.concatenate([o[s, :q_len[s]].ravel() for s in range(w.S)]) for o in outs)
-    for s in range(w.S):  # rows past q_len are not written
-        assert np.all(np.isnan(outs[0][s, q_len[s]:]))
-    m = oracle.diff_metrics(whole, got)
-    _say(f"split against whole: rel_l2={m['rel_l2']:.3e}")
-    assert m["rel_l2"] <= 1.1 * REL_L2, m
-    if mode in ("lengths", "causal"):
-        want = oracle.attention_for_workload(host, w.kv_type)
-        _check(np.concatenate([want[s, :q_len[s]].ravel() for s in range(w.S)]), got, "split")
+    got, whole, again = outs
+    assert np.array_equal(got, again, equal_nan=True)
+    n = int(max(c + r for c, r in zip(kv_len, q_len)))
+    want = oracle.flash_attn_ext(host["q"], np.ascontiguousarray(host["k"][:, :n]), np.ascontiguousarray(host["v"][:, :n]), kv,
+                                 np.ascontiguousarray(mask[..., :n]).view(np.uint16), max_bias=bias, logit_softcap=cap)
+    for s, r in enumerate(q_len):
+        assert np.all(np.isnan(got[s, r:]))  # rows past q_len are not written
+        if r == 0:
+            continue
+        for h in range(H):
+            _check(want[s, :r, h], got[s, :r, h], f"stream {s} head {h}")
+        m = oracle.diff_metrics(whole[s, :r], got[s, :r])
+        _say(f"stream {s}, split against whole: rel_l2={m['rel_l2']:.3e}")
+        assert m["rel_l2"] <= SPLIT_REL_L2, m
+
+
+def test_split_calls_of_two_streams_on_one_handle(fa):
+    """One handle, prompts of different streams in turn on two streams that run at once: every output is the
+    one its call gives alone."""
+    ws = [wl.Workload("two streams", 0x51A7_5600 + i, 1, [n], [r], D=d)
+          for i, (n, r, d) in enumerate(((6000, 40, 256), (5000, 64, 128)))]
+    devs = [wl.to_device(wl.make_host(w)) for w in ws]
+
+    def call(i):
+        out = torch.empty((1, ws[i].n_q, ws[i].H, ws[i].D), dtype=torch.float32, device="cuda")
+        d = devs[i]
+        fa(d["q"], d["k"], d["v"], out, kv_len=d["kv_len"], q_len=d["q_len"])
+        return out
+
+    _say("two streams, one handle")
+    alone = [call(i) for i in range(2)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = []
+    for _ in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                outs.append((i, call(i)))
+    torch.cuda.synchronize()
+    for i, out in outs:
+        assert torch.equal(out, alone[i])
 
 
 @pytest.mark.parametrize("D", [128, 256])
@@ -301,22 +355,27 @@ def test_split_in_the_fixed_scratch(fa):
 
 @pytest.mark.parametrize("D", [128, 256])
 @pytest.mark.parametrize("cached", [0, 87, 216, 3000])
-def test_shares_follow_the_cells_in_use(fa, cached, D):
+@pytest.mark.parametrize("masked", [False, True])
+def test_shares_follow_the_cells_in_use(fa, masked, cached, D):
     """A split launch is sized for the cache (16384 cells, NaN past the stream's); the cells in use decide
     how many work-groups share them, at least 128 cells each (40 rows behind 216 cells: two shares), and
-    the others write nothing.  With one share the sums are left alone and the output is the unsplit
+    the others write nothing, also where a llama mask's lengths are taken from the mask.  With one share the sums are left alone and the output is the unsplit
     call's bit for bit; always against the oracle."""
-    _say(f"short stream in a long cache: cached={cached} D={D}")
+    _say(f"short stream in a long cache: cached={cached} D={D} masked={masked}")
     w = wl.Workload("short stream", 0x51A7_5500 + cached + D, 1, [cached], [40], D=D)
     host = wl.make_host(w)
     dev = wl.to_device(host)
     k, v = (torch.full((1, 16384, w.Hkv, D), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
     for x, c in ((k, dev["k"]), (v, dev["v"])):
         x[:, :cached + 40] = c.view(torch.float16)[:, :cached + 40]
+    mask = None
+    if masked:
+        mask = torch.from_numpy(wl.kq_mask(16384, 40, w.kv_len, w.q_len)).view(torch.float16).cuda()
     outs = []
     for split in (True, False):
         out = torch.full((1, 40, w.H, D), float("nan"), dtype=torch.float32, device="cuda")
-        p = fa.params(dev["q"], k, v, out, kv_len=dev["kv_len"], q_len=dev["q_len"])
+        p = fa.params(dev["q"], k, v, out, kv_len=dev["kv_len"], q_len=dev["q_len"],
+                      mask_mode=sa.MASK_EXPLICIT if masked else sa.MASK_BLOCK_CAUSAL, mask=mask)
         least, full = _sizes(fa, p)
         ws = torch.full((full if split else least,), 0xA5, dtype=torch.uint8, device="cuda")
         _forward(fa, p, split, ws)
