@@ -411,7 +411,7 @@ class FlashAttnExt:
         among work-groups that leave sums in a workspace of the call's own (another order of the
         sums, so results agree with the unsplit call's to rounding).  None: eager calls on the
         current stream do, on a buffer from torch's allocator; captured ones, and those with an
-        explicit ``stream``, ``workspace``, ``bounded_workspace`` or ``noalloc``, do not.  True: those too -- the given
+        explicit ``stream``, ``workspace`` or ``noalloc``, do not.  True: those too -- the given
         workspace (or the fixed scratch) is this call's alone while it runs, or the capture is
         torch.cuda.graph's, whose memory pool gives the buffer.  False: never."""
         import torch
@@ -433,9 +433,8 @@ class FlashAttnExt:
         if rc == OK:
             if workspace is not None:
                 ws = workspace
-            elif least.value < n.value and (split_prefill or (
-                    split_prefill is None and stream is None and not bounded_workspace and
-                    not torch.cuda.is_current_stream_capturing())):
+            elif least.value < n.value and (split_prefill or (split_prefill is None and stream is None and
+                                                              not torch.cuda.is_current_stream_capturing())):
                 # the call's own until its kernels are queued (threads that share the stream may queue
                 # theirs in between), then the allocator's, which reuses it in this stream's order
                 ws = torch.empty(n.value, dtype=torch.uint8, device=self.device)

@@ -128,17 +128,6 @@ def test_who_splits(handle):
         _call(fa, split_prefill=True, stream=STREAM + 8)
 
 
-@pytest.mark.parametrize("q8", [False, True])
-def test_a_bounded_workspace_stays_a_token(handle, q8):
-    """bounded_workspace asks for the token that an unsplit prefill needs, whatever the cache."""
-    fa, state = handle
-    sizes = []
-    state["launch"] = lambda p: sizes.append(p.workspace_bytes)
-    for n_kv in (1024, 4096, 32768):
-        _call(fa, n_kv=n_kv, q8=q8, bounded_workspace=True)
-    assert max(sizes) <= 4096 and _held(fa) <= 4096
-
-
 def test_views_hold_what_they_are_given():
     """The packed view against the fields one by one: Python and numpy integers, a null pointer, the
     extents and strides of permuted and sliced tensors."""
