@@ -114,6 +114,11 @@ int attention_descriptors() {
                 std::fprintf(stderr, "workspace %zu\n", ws);
                 return -1;
             }
+            size_t least = 0, split = 0;  // without and with the split of prefill row blocks
+            if (sixi_attn_workspace_range(&p, &least, &split) != SIXI_OK || least != ws || split < ws || split % 256) {
+                std::fprintf(stderr, "workspace %zu, range %zu .. %zu\n", ws, least, split);
+                return -1;
+            }
         }
         (void)sixi_attn_strerror(rc);
     }
