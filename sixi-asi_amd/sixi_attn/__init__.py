@@ -282,7 +282,7 @@ assert _VIEW.size == ctypes.sizeof(SixiView)
 
 def make_view(data_ptr: int, type_id: int, ne, nb) -> SixiView:
     # (packed at once: ten conversions through the fields, and a tensor method for each stride and extent in
-    # view_of, took 8 of the 27 us of host time of a call with four views)
+    # view_of, made half of the host time of a call with four views)
     return SixiView.from_buffer_copy(_VIEW.pack(data_ptr or 0, type_id, 0, int(ne[0]), int(ne[1]), int(ne[2]), int(ne[3]),
                                                 int(nb[0]), int(nb[1]), int(nb[2]), int(nb[3])))
 
@@ -302,25 +302,26 @@ def view_of(t, type_id: Optional[int] = None, head_dim: Optional[int] = None,
     (Q, K, V as llama.cpp permutes them); False: the plain reversal (out, mask).
     For q8_0 pass a uint8 tensor whose last dim holds the packed blocks and ``head_dim``.
     """
-    if t.dim() != 4:
+    shape = t.shape
+    if len(shape) != 4:
         raise ValueError("expected a 4-d tensor")
     es = t.element_size()
-    order = (3, 1, 2, 0) if tokens_heads else (3, 2, 1, 0)
-    strides, shape = t.stride(), t.shape
-    nb = [strides[i] * es for i in order]
-    ne = [shape[i] for i in order]
+    n3, n1, n2, n0 = shape
+    b3, b1, b2, b0 = t.stride()
+    if not tokens_heads:
+        n1, n2, b1, b2 = n2, n1, b2, b1
+    b0 *= es
     if type_id is None:
         type_id = _float_types()[t.dtype]
     if type_id == TYPE_Q8_0:
         import torch
 
-        if t.dtype != torch.uint8 or head_dim is None or t.shape[-1] != head_dim // 32 * 34:
+        if t.dtype != torch.uint8 or head_dim is None or n0 != head_dim // 32 * 34:
             raise ValueError("q8_0 view needs a uint8 tensor of D/32*34 bytes per row and head_dim")
-        if t.stride(-1) != 1:
+        if b0 != 1:
             raise ValueError("q8_0 rows must be contiguous")
-        ne[0] = head_dim
-        nb[0] = 34
-    return make_view(t.data_ptr(), type_id, ne, nb)
+        n0, b0 = head_dim, 34
+    return SixiView.from_buffer_copy(_VIEW.pack(t.data_ptr(), type_id, 0, n0, n1, n2, n3, b0, b1 * es, b2 * es, b3 * es))
 
 
 class FlashAttnExt:
@@ -361,22 +362,25 @@ class FlashAttnExt:
         p.k = view_of(k, kvt, D if kvt == TYPE_Q8_0 else None)
         p.v = view_of(v, kvt, D if kvt == TYPE_Q8_0 else None)
         p.out = view_of(out, tokens_heads=False)
-        p.kv_len = kv_len.data_ptr() if kv_len is not None else None
-        p.q_len = q_len.data_ptr() if q_len is not None else None
+        if kv_len is not None:
+            p.kv_len = kv_len.data_ptr()
+        if q_len is not None:
+            p.q_len = q_len.data_ptr()
         p.mask_mode = mask_mode
-        p.flags = FLAG_BOUNDED_WORKSPACE if bounded_workspace else 0
-        if split_prefill:
-            p.flags |= FLAG_SPLIT_PREFILL
+        p.flags = ((FLAG_BOUNDED_WORKSPACE if bounded_workspace else 0) | (FLAG_SPLIT_PREFILL if split_prefill else 0) |
+                   (FLAG_GATE if gate is not None else 0))
         if gate is not None:
-            p.flags |= FLAG_GATE
             p.gate_qg = view_of(gate, tokens_heads=False)
         if mask is not None:
             # mask tensor [S or 1, 1, n_q_pad, n_kv] f16
             p.mask = view_of(mask, TYPE_F16, tokens_heads=False)
         p.scale = 1.0 / math.sqrt(D) if scale is None else scale
-        p.max_bias = max_bias
-        p.logit_softcap = logit_softcap
-        p.stream = stream
+        if max_bias:
+            p.max_bias = max_bias
+        if logit_softcap:
+            p.logit_softcap = logit_softcap
+        if stream is not None:
+            p.stream = stream
         if page_table is not None:
             p.page_table = page_table.data_ptr()
             p.page_table_stride = page_table.stride(0)
