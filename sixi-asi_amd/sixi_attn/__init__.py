@@ -329,9 +329,9 @@ class FlashAttnExt:
 
     Keeps a device workspace (grown on demand) so repeated calls allocate nothing; prefill calls that
     split their row blocks over idle CUs take one of their own from torch's allocator, so that they may
-    overlap other calls (``split_prefill`` of :meth:`__call__`).  A buffer that a larger call supersedes stays allocated for the life of the object, so a HIP graph
-    captured over an earlier call still owns the memory its kernels write.  A caller may
-    also pass its own ``workspace`` (a uint8 device tensor of at least
+    overlap other calls (``split_prefill`` of :meth:`__call__`).  A buffer that a larger call supersedes
+    stays allocated for the life of the object, so a HIP graph captured over an earlier call still owns
+    the memory its kernels write.  A caller may also pass its own ``workspace`` (a uint8 device tensor of at least
     :meth:`workspace_bytes`), e.g. one sized once before capture.
     """
 
